@@ -113,6 +113,11 @@ int tr_unpack_int4_pairs(const void* packed, void* qweight, void* scale, void* m
 int tr_dequant_int4(const void* qweight, const void* scale, const void* mn, void* out, int N, int K,
                     int group, int scale_dtype, void* stream);
 
+/* tr_dequant_int4 straight from the quad layout (pairs: the pair layout; rows come out in the engine's
+ * order). as_bf16 rounds an fp16-scale weight once more, to bf16; otherwise out is in the scale dtype. */
+int tr_dequant_packed(const void* packed, void* out, int N, int K, int scale_dtype, int pairs, int as_bf16,
+                      void* stream);
+
 /* ---------------------------------------------------------------- verify accept / commit
  *
  * logits bf16 [M, V] (1 <= M <= 32, 64 <= V <= 262144); tokens int64. `ws` is the accept

@@ -18,21 +18,8 @@
 // of an M = 1 call is bit-identical to row i of an M = 16 call (the property the reference's
 // tests/test_marlin.py:42-52 checks for Marlin), and likewise within M = 17..32.
 //
-// Weight layout ("quad layout", made once at load time by tr_pack_int4): the K/128 groups of a
-// 16-row strip are padded to a multiple of four (padding groups have zero codes, scale and min,
-// so they contribute exactly 0) and stored as quads of four groups, 4352 bytes each
-// (34 cache lines of 128 B, so no line is shared by two loads):
-//   packed[N/16][Gp/4][4352]
-//   bytes [1024 t, 1024 t + 1024): the codes of group 4 q + t. Lane l's 16 bytes at 16 l hold
-//     row l % 16 of the group as four 32-bit words; word j covers k0 = 32 j + 8 (l/16) .. k0 + 7
-//     (so MFMA j contracts k in [32 j, 32 j + 32) and the matching activations of one row are 64
-//     contiguous bytes) with code k0 + 2p in nibble p and k0 + 2p + 1 in
-//     nibble p + 4 (p = 0..3), so (w >> 4p) & 0x000F000F is the bf16 pair (k0 + 2p, k0 + 2p + 1)
-//     once the exponent is set.
-//   bytes [4096, 4352): row i's scale (low 16 bits) and min (high 16 bits) of group 4 q + t at
-//     4096 + 16 i + 4 t, so one 16-byte load gives a lane its row's parameters for all four groups.
-// A wave reads one strip's four groups with four 16-byte loads per lane plus one 16-byte load
-// of parameters, all at one scalar offset.
+// Weight layout: int4_layout.h. A wave reads one strip's four groups with four 16-byte loads per
+// lane plus one 16-byte load of parameters, all at one scalar offset.
 //
 // Work split ("activation-stationary"): a workgroup owns every grid_n-th strip and a K slot; each
 // of its W waves owns one K block of GW groups (GW = 4 for M <= 16, 2 above), loads that
@@ -42,6 +29,7 @@
 // [S, M, N] buffer (the contract of the reference's partials(), tokenrush/quant.py:381-391,
 // tokenrush/marlin.py:158-168) or a workspace the last-arriving slot reduces into bf16.
 #include "accept_common.h"
+#include "int4_layout.h"
 
 #include <mutex>
 
@@ -68,24 +56,13 @@ __device__ unsigned long long tr_tl_buf[kTlBlocks * 16 * kTlMarks];
   } while (0)
 #endif
 
-constexpr int kGroup = 128;
-constexpr int kQuad = 4;                          // groups per quad
-constexpr int kCodeBytes = 1024;                  // one group's codes for 16 rows
-constexpr int kSmOff = kQuad * kCodeBytes;        // parameters of the quad's groups
-constexpr int kQuadBytes = kSmOff + 16 * kQuad * 4;  // 4352 = 34 x 128 B
 constexpr int kWsCounterStride = 32;  // ints between workspace counters: one per 128-byte line
                                       // (agent-scope atomics on one line serialize)
 constexpr int kTailE = 4;      // last-arriver slot sum: outputs per thread per pass
 constexpr int kTailS = 2;      // and partial slots loaded per step
 constexpr int kMaxWaves = 12;   // 768 threads: leaves ~170 VGPRs per lane (3 waves per SIMD)
 
-// Groups of a K-long row after padding to whole quads.
-__host__ __device__ __forceinline__ int padded_groups(int K) { return (K / kGroup + kQuad - 1) / kQuad * kQuad; }
-
 enum { OUT_BF16 = 0, OUT_PARTIAL = 1, OUT_BF16_VIA_WS = 2 };
-
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 // One wave's GW groups of one strip: this lane's 16 code bytes per group and its row's
 // scale | min << 16 per group.
@@ -119,16 +96,6 @@ __device__ __forceinline__ void load_strip(Strip<GW>& t, __amdgpu_buffer_rsrc_t 
     const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, lane_off + gw * kCodeBytes, soff, 2 /* nt */);
     t.w[gw] = make_uint4(v.x, v.y, v.z, v.w);
   }
-}
-
-// Scale of a (scale | min << 16) word, fp32.
-template <bool F16S>
-__device__ __forceinline__ float sm_scale(uint32_t sm) {
-  return F16S ? f16_bits_to_f32(sm & 0xFFFFu) : __uint_as_float(sm << 16);
-}
-template <bool F16S>
-__device__ __forceinline__ float sm_min(uint32_t sm) {
-  return F16S ? f16_bits_to_f32(sm >> 16) : __uint_as_float(sm & 0xFFFF0000u);
 }
 
 // E = sum over the group of x * (128 + q), then acc += s * E. The group's other term,
@@ -632,120 +599,6 @@ __global__ __launch_bounds__(256) void slot_sum_kernel(const float* __restrict__
   }
 }
 
-// ----------------------------------------------------------------------------- layout kernels
-
-// Engine packing (uint8 [N, K/2], element 2j in the low nibble of byte j; tokenrush/quant.py:9-10)
-// plus scale/min [N, K/128] -> quad layout. One thread per output 32-bit word (1088 per quad);
-// padding groups are written as zeros.
-// Engine row of packed row i (0..15) of strip `strip`: identity, or for the gate/up pair layout
-// (F = N / 2 > 0) gate row 8 strip + i for i < 8 and up row F + 8 strip + i - 8 otherwise.
-__host__ __device__ __forceinline__ size_t src_row(size_t strip, int i, int F) {
-  return F > 0 ? (i < 8 ? 8 * strip + i : (size_t)F + 8 * strip + (i - 8)) : 16 * strip + i;
-}
-
-__global__ void pack_kernel(const uint32_t* __restrict__ q, const uint16_t* __restrict__ scale,
-                            const uint16_t* __restrict__ mn, uint32_t* __restrict__ packed, int N, int K, int F) {
-  const int G = K / kGroup, nq = padded_groups(K) / kQuad;
-  constexpr int kWords = kQuadBytes / 4;
-  const size_t total = (size_t)N / 16 * nq * kWords;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
-    const int d = i % kWords;
-    const size_t quad = i / kWords;
-    const size_t strip = quad / nq;
-    const int q0 = (int)(quad % nq) * kQuad;
-    if (d >= kSmOff / 4) {
-      const int e = d - kSmOff / 4, g = q0 + (e & 3);
-      const size_t n = src_row(strip, e >> 2, F);
-      packed[i] = g < G ? (uint32_t)scale[n * G + g] | ((uint32_t)mn[n * G + g] << 16) : 0u;
-      continue;
-    }
-    const int g = q0 + d / 256, j = d & 3, lane = (d & 255) >> 2;
-    if (g >= G) {
-      packed[i] = 0u;
-      continue;
-    }
-    const size_t n = src_row(strip, lane & 15, F);
-    const int k0 = g * kGroup + 32 * j + 8 * (lane >> 4);
-    const uint32_t u = q[(n * K + k0) / 8];  // bytes b0..b3 = codes k0..k0+7
-    uint32_t w = 0;
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const uint32_t b = (u >> (8 * p)) & 0xFF;
-      w |= (b & 0xF) << (4 * p);
-      w |= (b >> 4) << (16 + 4 * p);
-    }
-    packed[i] = w;
-  }
-}
-
-// Quad layout -> engine packing and scale/min (the inverse of pack_kernel; padding is dropped).
-__global__ void unpack_kernel(const uint32_t* __restrict__ packed, uint32_t* __restrict__ q,
-                              uint16_t* __restrict__ scale, uint16_t* __restrict__ mn, int N, int K, int F) {
-  const int G = K / kGroup, nq = padded_groups(K) / kQuad;
-  constexpr int kWords = kQuadBytes / 4;
-  const size_t total = (size_t)N / 16 * nq * kWords;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
-    const int d = i % kWords;
-    const size_t quad = i / kWords;
-    const size_t strip = quad / nq;
-    const int q0 = (int)(quad % nq) * kQuad;
-    const uint32_t w = packed[i];
-    if (d >= kSmOff / 4) {
-      const int e = d - kSmOff / 4, g = q0 + (e & 3);
-      if (g >= G) continue;
-      const size_t n = src_row(strip, e >> 2, F);
-      scale[n * G + g] = (uint16_t)(w & 0xFFFF);
-      mn[n * G + g] = (uint16_t)(w >> 16);
-      continue;
-    }
-    const int g = q0 + d / 256, j = d & 3, lane = (d & 255) >> 2;
-    if (g >= G) continue;
-    const size_t n = src_row(strip, lane & 15, F);
-    const int k0 = g * kGroup + 32 * j + 8 * (lane >> 4);
-    uint32_t u = 0;
-#pragma unroll
-    for (int p = 0; p < 4; ++p) {
-      const uint32_t lo = (w >> (4 * p)) & 0xF, hi = (w >> (16 + 4 * p)) & 0xF;
-      u |= (lo | (hi << 4)) << (8 * p);
-    }
-    q[(n * K + k0) / 8] = u;
-  }
-}
-
-// dequantize_int4 (tokenrush/quant.py:47-53): w = round(round(q * s) + m), two roundings, from the
-// engine packing. One thread per pair of elements (one byte).
-template <bool F16S>
-__global__ void dequant_kernel(const uint8_t* __restrict__ q, const uint16_t* __restrict__ scale,
-                               const uint16_t* __restrict__ mn, uint32_t* __restrict__ out, int N, int K) {
-  const int G = K / kGroup;
-  const size_t total = (size_t)N * K / 2;
-  for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < total; i += (size_t)gridDim.x * blockDim.x) {
-    const size_t n = i / (K / 2);
-    const int k = (int)(i % (K / 2)) * 2;
-    const size_t gi = n * G + k / kGroup;
-    // bf16 parameters: torch's in-place bf16 mul then add. fp16 parameters (the benchmark
-    // format): the same two roundings in fp16, output fp16.
-    const float s = F16S ? f16_bits_to_f32(scale[gi]) : bf16_bits_to_f32(scale[gi]);
-    const float m = F16S ? f16_bits_to_f32(mn[gi]) : bf16_bits_to_f32(mn[gi]);
-    const uint32_t b = q[i];
-    uint32_t r = 0;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const float code = (float)((b >> (4 * h)) & 0xF);
-      uint32_t bits;
-      if (F16S) {
-        const float t = (float)(_Float16)(code * s);
-        bits = __builtin_bit_cast(uint16_t, (_Float16)(t + m));
-      } else {
-        const float t = bf16_bits_to_f32(f32_to_bf16_bits(code * s));
-        bits = f32_to_bf16_bits(t + m);
-      }
-      r |= bits << (16 * h);
-    }
-    out[i] = r;
-  }
-}
-
 }  // namespace tr
 
 // ----------------------------------------------------------------------------- C ABI
@@ -755,14 +608,6 @@ namespace {
 
 constexpr int kCUs = 256;          // MI355X compute units
 
-// Bytes of the quad layout of an N x K weight.
-size_t packed_bytes(int N, int K) { return (size_t)N / 16 * (padded_groups(K) / kQuad) * kQuadBytes; }
-
-// Shapes the kernels take: whole 16-row strips and 128-wide groups, and a packed weight that
-// 32-bit buffer offsets address.
-bool shape_ok(int N, int K) {
-  return N > 0 && K > 0 && N % 16 == 0 && K % kGroup == 0 && packed_bytes(N, K) < ((size_t)1 << 31);
-}
 constexpr int kWavesPerCU = 12;    // occupancy of the GEMM kernel (about 150 VGPRs per lane)
 constexpr size_t kLdsBudget = 64 * 1024;  // LDS of the reduction ring
 constexpr size_t kLdsMax = 152 * 1024;    // dynamic LDS of one workgroup: gfx950's 160 KB less the kernel's static LDS
@@ -887,8 +732,6 @@ int tr_gemm_plan(int N, int K, int M, int* S, int* W, int* R) {
   *R = p.R;
   return TR_OK;
 }
-
-size_t tr_packed_bytes(int N, int K) { return shape_ok(N, K) ? packed_bytes(N, K) : 0; }
 
 int tr_partial_slots(int N, int K, int M) {
   Plan p;
@@ -1090,66 +933,6 @@ int tr_int4_gemm(const void* x, const void* packed, void* out, void* partials, v
                  void* stream) {
   return tr_int4_gemm_ex(x, packed, out, partials, workspace, workspace_bytes, M, N, K, group, scale_dtype,
                          partials ? n_slots : 0, 0, stream);
-}
-
-static int grid_for(size_t work) {
-  size_t b = (work + 255) / 256;
-  if (b > 65536) b = 65536;
-  if (b < 1) b = 1;
-  return (int)b;
-}
-
-static int pack_impl(const void* qweight, const void* scale, const void* mn, void* packed, int N, int K, int F,
-                     void* stream) {
-  if (!qweight || !scale || !mn || !packed) return TR_ERR_ARG;
-  if (!shape_ok(N, K) || (F && N % 32)) return TR_ERR_SHAPE;
-  const size_t total = packed_bytes(N, K) / 4;
-  hipLaunchKernelGGL(pack_kernel, dim3(grid_for(total)), dim3(256), 0, (hipStream_t)stream, (const uint32_t*)qweight,
-                     (const uint16_t*)scale, (const uint16_t*)mn, (uint32_t*)packed, N, K, F);
-  return hipGetLastError() == hipSuccess ? TR_OK : TR_ERR_LAUNCH;
-}
-
-static int unpack_impl(const void* packed, void* qweight, void* scale, void* mn, int N, int K, int F, void* stream) {
-  if (!qweight || !packed || !scale || !mn) return TR_ERR_ARG;
-  if (!shape_ok(N, K) || (F && N % 32)) return TR_ERR_SHAPE;
-  const size_t total = packed_bytes(N, K) / 4;
-  hipLaunchKernelGGL(unpack_kernel, dim3(grid_for(total)), dim3(256), 0, (hipStream_t)stream,
-                     (const uint32_t*)packed, (uint32_t*)qweight, (uint16_t*)scale, (uint16_t*)mn, N, K, F);
-  return hipGetLastError() == hipSuccess ? TR_OK : TR_ERR_LAUNCH;
-}
-
-int tr_pack_int4(const void* qweight, const void* scale, const void* mn, void* packed, int N, int K, void* stream) {
-  return pack_impl(qweight, scale, mn, packed, N, K, 0, stream);
-}
-
-int tr_unpack_int4(const void* packed, void* qweight, void* scale, void* mn, int N, int K, void* stream) {
-  return unpack_impl(packed, qweight, scale, mn, N, K, 0, stream);
-}
-
-int tr_pack_int4_pairs(const void* qweight, const void* scale, const void* mn, void* packed, int N, int K,
-                       void* stream) {
-  return pack_impl(qweight, scale, mn, packed, N, K, N / 2, stream);
-}
-
-int tr_unpack_int4_pairs(const void* packed, void* qweight, void* scale, void* mn, int N, int K, void* stream) {
-  return unpack_impl(packed, qweight, scale, mn, N, K, N / 2, stream);
-}
-
-int tr_dequant_int4(const void* qweight, const void* scale, const void* mn, void* out, int N, int K, int group,
-                    int scale_dtype, void* stream) {
-  if (!qweight || !scale || !mn || !out) return TR_ERR_ARG;
-  if (group != kGroup) return TR_ERR_CONFIG;
-  if (N <= 0 || K <= 0 || K % kGroup) return TR_ERR_SHAPE;
-  const size_t total = (size_t)N * K / 2;
-  if (scale_dtype == 1)
-    hipLaunchKernelGGL(dequant_kernel<true>, dim3(grid_for(total)), dim3(256), 0, (hipStream_t)stream,
-                       (const uint8_t*)qweight, (const uint16_t*)scale, (const uint16_t*)mn, (uint32_t*)out, N, K);
-  else if (scale_dtype == 0)
-    hipLaunchKernelGGL(dequant_kernel<false>, dim3(grid_for(total)), dim3(256), 0, (hipStream_t)stream,
-                       (const uint8_t*)qweight, (const uint16_t*)scale, (const uint16_t*)mn, (uint32_t*)out, N, K);
-  else
-    return TR_ERR_ARG;
-  return hipGetLastError() == hipSuccess ? TR_OK : TR_ERR_LAUNCH;
 }
 
 #ifdef TR_TIMELINE

@@ -288,3 +288,19 @@ def dequantize(qweight: torch.Tensor, scale: torch.Tensor, mn: torch.Tensor) -> 
     _lib.check(ext().tr_dequant_int4(_lib.ptr(q), _lib.ptr(s), _lib.ptr(m), _lib.ptr(out), N, K, K // s.shape[1],
                                      SCALE_DTYPES[s.dtype], _lib.stream_of(q)), "tr_dequant_int4")
     return out
+
+
+def dequantize_packed(B: torch.Tensor, s: torch.Tensor, K: int, pairs: bool = False, dtype=None) -> torch.Tensor:
+    """dequantize() straight from the quad layout (pack's B and s): dense [N, K] in the engine's row order,
+    in the scale dtype or, for dtype bfloat16, that product rounded to bf16."""
+    _lib.require_gpu(B)
+    N = B.shape[0] * 16
+    if padded_groups(K) != B.shape[1] * 4 or not B.is_contiguous():
+        raise RuntimeError(f"K = {K} does not match the packed weight ({B.shape[1]} quads per strip)")
+    dtype = s.dtype if dtype is None else dtype
+    if dtype not in (s.dtype, torch.bfloat16):
+        raise RuntimeError("dequantize_packed: the scale dtype or bfloat16")
+    out = torch.empty(N, K, dtype=dtype, device=B.device)
+    _lib.check(ext().tr_dequant_packed(_lib.ptr(B), _lib.ptr(out), N, K, SCALE_DTYPES[s.dtype], int(pairs),
+                                       int(dtype == torch.bfloat16), _lib.stream_of(B)), "tr_dequant_packed")
+    return out

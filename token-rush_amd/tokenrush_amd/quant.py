@@ -103,14 +103,20 @@ class QLinear:
         """A QLinear over the output rows `ids` (the truncated draft vocabulary)."""
         return QLinear(*(t.index_select(0, ids) for t in self.nibbles()), backend=self.backend, split_k=self.split_k)
 
-    def dequantize(self) -> torch.Tensor:
-        return dequantize_int4(*self.nibbles())
+    def dequantize(self, dtype=None) -> torch.Tensor:
+        """Dense [N, K] in the scale dtype (then rounded to `dtype` when given)."""
+        if self.backend != "gfx950":
+            w = dequantize_int4(self.qweight, self.scale, self.mn)
+        else:
+            direct = dtype if dtype == torch.bfloat16 else None
+            w = gfx950.dequantize_packed(self.B, self.s, self.shape_[1], self.layout == "gate_up", direct)
+        return w if dtype is None else w.to(dtype)
 
     def __call__(self, x: torch.Tensor, out: torch.Tensor = None) -> torch.Tensor:
         """x [T, K] -> [T, N]; out (bf16 [T, N], contiguous) receives the product when given."""
         T = x.shape[0]
         if self.backend == "dequant" or T > MAX_ROWS:
-            y = F.linear(x, self.dequantize().to(x.dtype))
+            y = F.linear(x, self.dequantize(x.dtype))
         elif self.layout == "gate_up":
             y = gfx950.unpair(gfx950.mul(x.contiguous(), self.B, self.s))
         else:
