@@ -88,6 +88,16 @@ int tr_partial_slots(int N, int K, int M);
  * Replaces: the lock + fp32 reduce buffer sizing of marlin.workspaces (tokenrush/marlin.py:121-135). */
 size_t tr_gemm_workspace_bytes(int N, int K, int M);
 
+/* Prompts: the same product for T > 32 rows (x [T, K], 16-byte aligned; T <= 65535, 2 T K < 2^31) on a
+ * packed weight. mode 0: a plain weight, out [T, N]; 1: a pair-layout [gate; up] weight, out [T, N] in the
+ * engine's column order; 2: a pair-layout weight, out [T, N/2] = silu(bf16(gate)) * bf16(up). workspace: scratch of
+ * tr_prompt_workspace_bytes(T, N, K) bytes (0: unsupported shape), any contents; calls that overlap must not
+ * share it. Two launches, or three when the plan splits K.
+ * Replaces: the T > 32 path of QLinear (tokenrush/quant.py:373-374: dequantize, then a dense matmul). */
+size_t tr_prompt_workspace_bytes(int T, int N, int K);
+int tr_int4_gemm_prompt(const void* x, const void* packed, void* out, void* workspace, size_t workspace_bytes, int T,
+                        int N, int K, int group, int scale_dtype, int mode, void* stream);
+
 /* Bytes of the quad layout of an N x K weight (0: unsupported shape -- N % 16, K % 128, or a
  * packed size of 2 GiB or more). Host only. */
 size_t tr_packed_bytes(int N, int K);

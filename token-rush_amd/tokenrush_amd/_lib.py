@@ -38,6 +38,8 @@ SIGNATURES = {
     "tr_pack_int4_pairs": (_I, [_P, _P, _P, _P, _I, _I, _P]),
     "tr_unpack_int4_pairs": (_I, [_P, _P, _P, _P, _I, _I, _P]),
     "tr_dequant_int4": (_I, [_P, _P, _P, _P, _I, _I, _I, _I, _P]),
+    "tr_prompt_workspace_bytes": (_S, [_I, _I, _I]),
+    "tr_int4_gemm_prompt": (_I, [_P, _P, _P, _P, _S, _I, _I, _I, _I, _I, _I, _P]),
     "tr_dequant_packed": (_I, [_P, _P, _I, _I, _I, _I, _I, _P]),
     "tr_accept_workspace_bytes": (_S, [_I, _I]),
     "tr_lm_head_workspace_bytes": (_S, [_I, _I, _I]),

@@ -249,6 +249,30 @@ def mul_silu(x: torch.Tensor, B: torch.Tensor, s: torch.Tensor):
     return y
 
 
+PROMPT_ROWS, PROMPT_PAIRS, PROMPT_SILU = 0, 1, 2   # output forms of mul_prompt
+
+
+def mul_prompt(x: torch.Tensor, B: torch.Tensor, s: torch.Tensor, mode: int = PROMPT_ROWS):
+    """x [T, K] bf16 (T > 32) -> [T, N] bf16; B a plain weight, or a pair-layout [gate; up] weight whose
+    product comes out in the engine's column order (PROMPT_PAIRS) or as silu(gate) * up [T, N/2] (PROMPT_SILU).
+    No weight is rounded to bf16 first, unlike a product with the dense copy; a row of x that holds an
+    infinity comes out NaN, as in mul(). The scratch is this call's own: calls on several streams may overlap."""
+    T, K = x.shape
+    N = B.shape[0] * 16
+    need = int(ext().tr_prompt_workspace_bytes(T, N, K))
+    shape = (T, N // 2 if mode == PROMPT_SILU else N)
+    if x.dtype != torch.bfloat16 or not x.is_contiguous() or not B.is_contiguous() or padded_groups(K) != B.shape[1] * 4 \
+            or need == 0:
+        raise RuntimeError(f"mul_prompt: problem shape (t={T}, n={N}, k={K}) not supported, or x not contiguous bf16")
+    _lib.require_gpu(x, B)
+    y = torch.empty(*shape, dtype=torch.bfloat16, device=x.device)
+    ws = torch.empty(need, dtype=torch.uint8, device=x.device)
+    rc = ext().tr_int4_gemm_prompt(_lib.ptr(x), _lib.ptr(B), _lib.ptr(y), _lib.ptr(ws), need, T, N, K, GROUP,
+                                   SCALE_DTYPES[s.dtype], mode, _lib.stream_of(x))
+    _lib.check(rc, f"tr_int4_gemm_prompt (t={T}, n={N}, k={K})")
+    return y
+
+
 _slots = {}
 
 

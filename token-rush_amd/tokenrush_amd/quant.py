@@ -20,7 +20,7 @@ from . import gfx950
 GROUP = 128
 BACKENDS = ("gfx950", "dequant")
 DEFAULT_BACKEND = "gfx950"
-MAX_ROWS = gfx950.MAX_ROWS        # beyond this T the prefill path (dequant + matmul) runs
+MAX_ROWS = gfx950.MAX_ROWS        # beyond this T a prompt path runs: the prompt GEMM, or dequant + matmul
 _ALIASES = {"marlin": "gfx950", "triton": "gfx950", "tinygemm": "gfx950"}
 
 
@@ -49,6 +49,26 @@ def dequantize_int4(packed, scale, mn) -> torch.Tensor:
     """-> [out, in] in the scale dtype: round(round(q * s) + m), the reference's two bf16
     roundings (quant.py:47-53), computed by the HIP dequant kernel."""
     return gfx950.dequantize(packed, scale, mn)
+
+
+def _prompt_kernel(T: int, N: int, K: int) -> bool:
+    """Whether T > MAX_ROWS rows go through the prompt GEMM on the packed weight rather than a dense copy of
+    it and the library matmul. The kernel saves the dense copy (2 N K bytes written, then read), the library
+    has the faster inner loop. Measured, us, kernel / dense: 7168 x 5120 47 / 67 at 256 rows, 60 / 58 at 384;
+    14336 x 5120 64 / 85 and 96 / 88; 34816 x 5120 142 / 200, 196 / 261 and 260 / 280 at 512, 320 / 349 at
+    640; 5120 x 17408 82 / 214, 112 / 166, 178 / 199. So 256 rows for every weight, and 512 where the dense
+    copy is far beyond what the caches hold."""
+    return T <= 256 or (T <= 512 and N * K >= 80_000_000)
+
+
+def _plain(x: torch.Tensor) -> bool:
+    """x is an ordinary device tensor outside autograd, autocast, function transforms and tracing: F.linear
+    would do nothing but the product."""
+    return (type(x) is torch.Tensor and x.is_cuda and x.dim() == 2 and x.dtype == torch.bfloat16
+            and not (x.requires_grad and torch.is_grad_enabled()) and not torch.is_autocast_enabled("cuda")
+            and not torch.compiler.is_compiling() and torch._C._get_tracing_state() is None
+            and torch._C._len_torch_dispatch_stack() == 0 and not torch._C._functorch.is_functorch_wrapped_tensor(x)
+            and torch.autograd.forward_ad._current_level < 0)
 
 
 class QLinear:
@@ -112,11 +132,24 @@ class QLinear:
             w = gfx950.dequantize_packed(self.B, self.s, self.shape_[1], self.layout == "gate_up", direct)
         return w if dtype is None else w.to(dtype)
 
+    def _prompt(self, x: torch.Tensor, mode: int):
+        """x's product through the prompt GEMM, or None where the dense path is the faster or only one."""
+        N, K = self.shape_
+        if self.backend != "gfx950" or not _plain(x) or x.shape[1] != K or x.device != self.B.device \
+                or not _prompt_kernel(x.shape[0], N, K):
+            return None
+        x = x.contiguous()
+        if x.data_ptr() % 16:
+            x = x.clone()
+        return gfx950.mul_prompt(x, self.B, self.s, mode)
+
     def __call__(self, x: torch.Tensor, out: torch.Tensor = None) -> torch.Tensor:
         """x [T, K] -> [T, N]; out (bf16 [T, N], contiguous) receives the product when given."""
         T = x.shape[0]
         if self.backend == "dequant" or T > MAX_ROWS:
-            y = F.linear(x, self.dequantize(x.dtype))
+            y = self._prompt(x, gfx950.PROMPT_PAIRS if self.layout == "gate_up" else gfx950.PROMPT_ROWS)
+            if y is None:
+                y = F.linear(x, self.dequantize(x.dtype))
         elif self.layout == "gate_up":
             y = gfx950.unpair(gfx950.mul(x.contiguous(), self.B, self.s))
         else:
@@ -127,8 +160,11 @@ class QLinear:
         """silu(gate) * up of this [gate; up] weight's product, [T, N/2] bf16: one fused launch
         for a "gate_up" layout, else the product followed by the activation kernel
         (tokenrush/model.py:156-160 with fused.py:67-87)."""
-        if self.layout == "gate_up" and x.shape[0] <= MAX_ROWS:
-            return gfx950.mul_silu(x.contiguous(), self.B, self.s)
+        if self.layout == "gate_up":
+            y = gfx950.mul_silu(x.contiguous(), self.B, self.s) if x.shape[0] <= MAX_ROWS else \
+                self._prompt(x, gfx950.PROMPT_SILU)
+            if y is not None:
+                return y
         from .fused import silu_mul
         return silu_mul(self(x))
 
