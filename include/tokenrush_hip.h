@@ -293,8 +293,8 @@ int tr_attn_prep(const void* qkv, int ld, const void* q_norm_w, const void* k_no
                  float* v_scale, int maxlen, void* q_out, int M, int HQ, int HKV, int D, float eps, void* stream);
 
 /* Flash-decoding of M (1..8) query tokens over cache rows 0..*pos + M - 1 (query t sees rows
- * <= *pos + t): nsplit key-range splits (two launches: split, then combine + sigmoid output gate
- * from qkv) -> out [M, HQ D] bf16. D == 256.
+ * <= *pos + t): up to nsplit key-range splits (fewer where they would not fit one workgroup per CU; two
+ * launches: split, then combine + sigmoid output gate from qkv) -> out [M, HQ D] bf16. D == 256.
  * Replaces: attn_decode_fused (tokenrush/fused.py:355-470: _attn_split_kernel + _attn_reduce_kernel). */
 int tr_attn_decode(const void* q, const void* qkv, int ld, const void* k_cache, const void* v_cache,
                    const float* k_scale, const float* v_scale, int maxlen, const int64_t* pos, void* out,
@@ -311,7 +311,7 @@ int tr_attn_prep_tree(const void* qkv, int ld, const void* q_norm_w, const void*
 
 /* Draft-tree flash-decoding, M (1..32) nodes: node t sees the committed rows < *pos and the new
  * rows *pos + i of its ancestors and itself (the ancestor mask). Otherwise as tr_attn_decode; the
- * query rows of a kv head run in groups of 64, one more grid dimension.
+ * query rows of a kv head run in groups of up to 48, one more grid dimension.
  * No counterpart in the reference; the per-node arithmetic is attn_decode_fused's (tokenrush/fused.py:355-470). */
 int tr_attn_decode_tree(const void* q, const void* qkv, int ld, const void* k_cache, const void* v_cache,
                         const float* k_scale, const float* v_scale, int maxlen, const int64_t* pos,

@@ -14,25 +14,40 @@
 //   summed before the value scale, P = bf16(p * vsc), acc += P v8;
 //   splits combined by their maxima; o = bf16(acc / l) * bf16(sigmoid(gate)), bf16 out.
 //
-// MI355X layout of the split kernel: one workgroup of four waves per (kv head, split); the
-// G * M query rows of the kv head (G = HQ / HKV query heads per token) are 16-row MFMA tiles,
-// one per wave. Keys stream through LDS 32 at a time: K dequantized to bf16 row-major, V
-// converted to bf16 and transposed (d-major) while it is written. Scores are computed transposed,
-// S^T = K Q^T (v_mfma_f32_16x16x32_bf16, Q^T stationary in registers), which leaves each lane
-// the scores of one query row for 8 keys: exactly the B operand of O^T = V^T P^T once the key
-// order inside the 32-key step is permuted the same way on the V^T side. Row maxima and sums
-// need two xor shuffles. Each wave keeps O^T for its 16 rows x 256 d in 64 registers.
+// MI355X layout of the split kernel: one workgroup of four waves per (kv head, split, group of up to 48 of
+// the G M query rows of the kv head, G = HQ / HKV). The waves take alternate 32-key blocks and each runs all
+// of the group's rows on its own block, straight from the cache rows in registers: no LDS and no barrier
+// between the blocks.
+//   S^T = K8 Q^T (v_mfma_f32_16x16x32_bf16): a lane's 16-byte load of a key row is the A operand of two MFMAs
+//   (fp8 is exact in bf16; the k index may run over the dims in any order that Q^T, held in LDS, shares); the
+//   key's scale multiplies the fp32 score. The lane then holds eight keys' scores of one query row, which is
+//   the B operand of O^T = V^T P^T for those keys. V: a lane loads 16 dims of its eight keys; byte e of the
+//   eight is the A operand of O^T tile e (dims 16 i + e), so V is transposed in registers, by v_perm_b32.
+//   Row maxima need two permlane swaps, row sums are made after the loop. After the last block the waves'
+//   (m, l, O^T) meet in LDS.
+// Each wave keeps O^T for up to 48 rows x 256 d in 192 AGPRs, one workgroup per CU, so the launch takes as
+// many splits as leave one workgroup per CU.
+//
+// Before, four waves converted each block into LDS together (two barriers and a transposed write per block)
+// and then held 16 query rows each: 2.4 us per 32 keys of a CU, whatever the rows. Split + combine, us
+// (24 / 4 heads): 1 token over 100k rows 87 -> 42, 4 tokens 90 -> 46 (208 MB, 4.9 TB/s in the split kernel),
+// 8 tokens 93 -> 54; over 8k rows 15.7 -> 12.6, 19.0 -> 16.4, 22.6 -> 21.0; a 32-node tree over 8k 37 -> 29.
+// Measured and not kept: a second block of K and V in flight in registers (M = 8 over 8k 22.3 us, 100k 61.6;
+// the copies cost more than the wait); key splits not rounded to four blocks (22.9 us at 8k); partial rows
+// stored whole through a transposing LDS read (22.6 us; the merge of a 16-row tile costs 2.3 us either way).
 #include "accept_common.h"
+
+#include <atomic>
 
 namespace tr {
 
 constexpr int kAttnD = 256;      // head dim
-constexpr int kAttnBlk = 32;     // keys per LDS block
+constexpr int kAttnBlk = 32;     // keys per block
 constexpr int kAttnMaxM = 8;     // query tokens per chain step
 constexpr int kAttnMaxTree = 32; // query tokens (nodes) per draft-tree step: one bit each in a mask word
 constexpr int kAttnWaves = 4;
-constexpr int kKPitch = kAttnD + 8;     // bf16 elements per K row in LDS
-constexpr int kVPitch = kAttnBlk + 4;   // bf16 elements per V^T row (one d) in LDS
+constexpr int kAttnTiles = 3;    // 16-row query tiles per workgroup, at most
+constexpr int kAttnCUs = 256;
 constexpr float kFp8Max = 448.f;
 constexpr float kLog2e = 1.4426950408889634f;  // scores are kept in log2 units: p = 2^(s - m)
 constexpr int kMaxSplit = 256;  // key-range splits of one flash-decoding call
@@ -61,21 +76,20 @@ __device__ __forceinline__ uint32_t f32_to_fp8(float x) {
 
 __device__ __forceinline__ float bf16r_a(float v) { return bf16_bits_to_f32(f32_to_bf16_bits(v)); }
 
-typedef float f32x2v __attribute__((ext_vector_type(2)));
+typedef uint32_t u32x4a __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x2v __attribute__((ext_vector_type(2)));
 // Two fp32 -> packed bf16 (round to nearest even, v_cvt_pk_bf16_f32).
 __device__ __forceinline__ uint32_t pk_bf16(float x, float y) {
   const bf16x2v r = {(__bf16)x, (__bf16)y};
   return __builtin_bit_cast(uint32_t, r);
 }
-// fp8 e4m3fn bytes 0,1 (hi = false) or 2,3 (hi = true) of w -> fp32, exact (v_cvt_pk_f32_fp8).
-__device__ __forceinline__ f32x2v fp8x2_to_f32(uint32_t w, bool hi) {
-  return hi ? __builtin_amdgcn_cvt_pk_f32_fp8(w, true) : __builtin_amdgcn_cvt_pk_f32_fp8(w, false);
-}
-// Exact fp8 -> bf16 of two values: the fp32 images have zero low halves.
-__device__ __forceinline__ uint32_t fp8x2_to_bf16(uint32_t w, bool hi) {
-  const f32x2v f = fp8x2_to_f32(w, hi);
-  return (__float_as_uint(f.x) >> 16) | (__float_as_uint(f.y) & 0xFFFF0000u);
+// Eight fp8 bytes -> bf16, exact (scale 1).
+__device__ __forceinline__ bf16x8 fp8x8_to_bf16(uint32_t lo, uint32_t hi) {
+  const uint4 v = make_uint4(__builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.f, false)),
+                             __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 1.f, true)),
+                             __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.f, false)),
+                             __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 1.f, true)));
+  return __builtin_bit_cast(bf16x8, v);
 }
 __device__ __forceinline__ float max_x16(float v) {
   const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -233,55 +247,32 @@ struct AttnSplitArgs {
   float scale;
 };
 
-template <bool TREE>
-__global__ __launch_bounds__(64 * kAttnWaves) void attn_split_kernel(AttnSplitArgs a) {
-  __shared__ __attribute__((aligned(16))) uint16_t Ks[kAttnBlk * kKPitch];
-  __shared__ __attribute__((aligned(16))) uint16_t Vt[kAttnD * kVPitch];
-  __shared__ float ksc[kAttnBlk], vsc[kAttnBlk];
+// Splits that hold keys: split s takes blocks s per .. of the nblk live blocks, per a multiple of the four
+// waves (a wave alone on a last block takes as long as four, and fewer splits mean fewer partials to combine).
+struct AttnRange {
+  int nblk, per;
+  __device__ __forceinline__ AttnRange(int64_t L, int nsplit) {
+    nblk = (int)((L + kAttnBlk - 1) / kAttnBlk);
+    per = ((nblk + nsplit - 1) / nsplit + kAttnWaves - 1) / kAttnWaves * kAttnWaves;
+  }
+  // split 0 always counts: it writes the empty partials of a call without live rows
+  __device__ __forceinline__ int used(int nsplit) const { return per > 0 ? max(1, min(nsplit, (nblk + per - 1) / per)) : 1; }
+};
+
+// T 16-row query tiles per workgroup; its four waves take alternate key blocks of the split.
+template <int T>
+__global__ __launch_bounds__(64 * kAttnWaves, 1) void attn_split_kernel(AttnSplitArgs a) {
+  extern __shared__ __attribute__((aligned(16))) float lds[];  // Q operands; after the loop each wave's O^T tile, then its (m, l)
   const int j = blockIdx.x / a.nsplit, s = blockIdx.x % a.nsplit;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int G = a.HQ / a.HKV;
-  const int gy = TREE ? (int)blockIdx.y : 0;  // row group (a chain's M * G rows fit one)
-  const int rows = G * a.M - 16 * kAttnWaves * gy;  // this workgroup's row group
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int i = lane & 15, o = lane >> 4;
+  const int G = a.HQ / a.HKV, rows = G * a.M;
+  const int tile0 = (int)blockIdx.y * T;
   const int64_t pos = *a.pos;
   const int64_t L = pos + a.M;
-  const int nblk = (int)((L + kAttnBlk - 1) / kAttnBlk);
-  const int per = (nblk + a.nsplit - 1) / a.nsplit;
-  const int b0 = s * per, b1 = min(b0 + per, nblk);
-  const bool computes = 16 * wave < rows;
-
-  // Q^T operand: lane l holds row 16 wave + l % 16, dims 8 (l / 16) + 32 jj .. + 7
-  const int row = 16 * wave + (lane & 15);
-  const bool rvalid = row < rows;
-  const int grow = 16 * kAttnWaves * gy + row;  // row of the kv head: query qi, head g
-  const int qi = rvalid ? grow / G : 0;
-  const int hq = j * G + (rvalid ? grow % G : 0);
-  uint4 qb[8];
-#pragma unroll
-  for (int jj = 0; jj < 8; ++jj)
-    qb[jj] = rvalid ? *(const uint4*)(a.q + ((size_t)qi * a.HQ + hq) * kAttnD + 8 * (lane >> 4) + 32 * jj)
-                    : make_uint4(0, 0, 0, 0);
-  // The new keys query qi sees: rows pos + i for the bits i of vis -- i <= qi for a chain, the
-  // node's ancestors and itself for a tree.
-  uint32_t vis = qi >= 31 ? ~0u : (2u << qi) - 1u;
-  const int64_t qlimit = pos + qi;  // a chain's last visible row
-  if (TREE) {
-    // the parents one per lane (one load for the wave), then the walk by shuffles
-    const int pl = lane > 0 && lane < a.M ? attn_tree_parent(a.parent, lane) : 0;
-    vis = 0;
-    int jn = qi;
-    for (int d = 0; d < kAttnMaxTree; ++d) {
-      vis |= 1u << jn;
-      jn = __shfl(pl, jn);  // the root's entry is 0
-      if (__all(jn == 0)) break;
-    }
-    vis |= 1u;  // the root: every node sees it
-  }
-
-  f32x4 acc[16];
-#pragma unroll
-  for (int dt = 0; dt < 16; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  float m_i = -INFINITY, l_i = 0.f;
+  const AttnRange range(L, a.nsplit);
+  const int b0 = s * range.per, b1 = min(b0 + range.per, range.nblk);
+  if (s >= range.used(a.nsplit)) return;
 
   // Cache reads go through buffer resources sized to the L live rows: rows past them, and the
   // prefetch past the split's last block, read zeros with no memory access and no branch.
@@ -294,149 +285,218 @@ __global__ __launch_bounds__(64 * kAttnWaves) void attn_split_kernel(AttnSplitAr
                                                      0x00020000);
   const auto vsr = __builtin_amdgcn_make_buffer_rsrc((void*)(a.v_scale + (size_t)j * a.maxlen), (short)0, liveL * 4,
                                                      0x00020000);
-  constexpr int kOob = 0x7FFFFFF0;
-  // fill roles: K: thread t loads key t / 8, dims 32 (t % 8) .. + 31; V: keys 4 (t % 8) .. + 3,
-  // dims 8 (t / 8) .. + 7; scales: threads 0..31 (V) and every 8th thread (K)
-  const int fk = tid >> 3, fkd = 32 * (tid & 7);
-  const int fv = 4 * (tid & 7), fvd = 8 * (tid >> 3);
-  typedef uint32_t u4 __attribute__((ext_vector_type(4)));
-  typedef uint32_t u2 __attribute__((ext_vector_type(2)));
-  u4 pk0, pk1;
-  u2 pv[4];
-  float psk, psv;
-  // the cache rows are read once per step: non-temporal, as the GEMM streams its weights
-  constexpr int kNt = 2;
-  auto fetch = [&](int blk, bool on) {
-    const int key0 = blk * kAttnBlk;
-    const int kk = key0 + fk;
-    pk0 = __builtin_amdgcn_raw_buffer_load_b128(krs, on ? kk * kAttnD + fkd : kOob, 0, kNt);
-    pk1 = __builtin_amdgcn_raw_buffer_load_b128(krs, on ? kk * kAttnD + fkd + 16 : kOob, 0, kNt);
-    psk = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(ksr, on ? kk * 4 : kOob, 0, kNt));
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      pv[i] = __builtin_amdgcn_raw_buffer_load_b64(vrs, on ? (key0 + fv + i) * kAttnD + fvd : kOob, 0, kNt);
-    psv = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(vsr, on && tid < kAttnBlk ? (key0 + tid) * 4 : kOob, 0, kNt));
-  };
-  fetch(b0, b0 < b1);
-  for (int blk = b0; blk < b1; ++blk) {
-    const int64_t key0 = (int64_t)blk * kAttnBlk;
-    __syncthreads();  // the previous block's LDS reads are done
-    {
-      const uint32_t kw[8] = {pk0.x, pk0.y, pk0.z, pk0.w, pk1.x, pk1.y, pk1.z, pk1.w};
-      const float sck = psk;
-      uint16_t* dst = Ks + fk * kKPitch + fkd;
-#pragma unroll
-      for (int q4 = 0; q4 < 4; ++q4) {
-        uint32_t o[4];
-#pragma unroll
-        for (int h = 0; h < 4; ++h) {
-          const f32x2v f = fp8x2_to_f32(kw[2 * q4 + h / 2], h & 1);
-          o[h] = pk_bf16(f.x * sck, f.y * sck);
-        }
-        *(uint4*)(dst + 8 * q4) = make_uint4(o[0], o[1], o[2], o[3]);
-      }
-      if ((tid & 7) == 0) ksc[fk] = sck;
-    }
-    {
-      // 4 keys x 8 dims -> 8 rows of V^T (4 keys each): byte e of key i is pv[i] byte e. One
-      // v_perm_b32 gathers byte e of two keys, one scaled conversion (scale 1: exact) makes the
-      // bf16 pair.
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const uint32_t sel = 0x0C0C0000u | ((4u + (e & 3)) << 8) | (uint32_t)(e & 3);  // b0 = lo[e], b1 = hi[e]
-        const uint32_t w01 = __builtin_amdgcn_perm(e < 4 ? pv[1].x : pv[1].y, e < 4 ? pv[0].x : pv[0].y, sel);
-        const uint32_t w23 = __builtin_amdgcn_perm(e < 4 ? pv[3].x : pv[3].y, e < 4 ? pv[2].x : pv[2].y, sel);
-        uint2 o;
-        o.x = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w01, 1.f, false));
-        o.y = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(w23, 1.f, false));
-        *(uint2*)(Vt + (fvd + e) * kVPitch + fv) = o;
-      }
-      if (tid < kAttnBlk) vsc[tid] = psv;
-    }
-    fetch(blk + 1, blk + 1 < b1);  // the next block's loads run under this block's compute
-    __syncthreads();
-    if (!computes) continue;
-    // S^T = K Q^T for the block's two 16-key tiles: lane gets keys 16 kt + 4 (l / 16) + r, row l % 16
-    f32x4 st[2];
+  constexpr uint32_t kOob = 0x7FFF0000u;
+  constexpr int kNt = 2;  // the cache rows are read once per step: non-temporal, as the GEMM streams its weights
+  // K: lane (i, o) loads key 16 kt + i, dims 64 c + 16 o .. + 15; V: keys 16 kt + 4 o + r, dims 16 i .. + 15;
+  // the scales of keys 16 kt + 4 o .. + 3
+  u32x4a kraw[2][4], vraw[2][4], ksv[2], vsv[2];
+  auto fetch_k = [&](int blk) {
+    const uint32_t base = blk < b1 ? (uint32_t)blk * kAttnBlk : kOob / kAttnD;
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt) {
-      f32x4 c = {0.f, 0.f, 0.f, 0.f};
-      const uint16_t* kr = Ks + (16 * kt + (lane & 15)) * kKPitch + 8 * (lane >> 4);
 #pragma unroll
-      for (int jj = 0; jj < 8; ++jj) {
-        const uint4 kv = *(const uint4*)(kr + 32 * jj);
-        c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, kv), __builtin_bit_cast(bf16x8, qb[jj]),
-                                                    c, 0, 0, 0);
+      for (int c = 0; c < 4; ++c)
+        kraw[kt][c] = __builtin_amdgcn_raw_buffer_load_b128(krs, (base + 16 * kt + i) * kAttnD + 16 * o + 64 * c, 0, kNt);
+      ksv[kt] = __builtin_amdgcn_raw_buffer_load_b128(ksr, (base + 16 * kt + 4 * o) * 4, 0, kNt);
+    }
+  };
+  auto fetch_v = [&](int blk) {
+    const uint32_t base = blk < b1 ? (uint32_t)blk * kAttnBlk : kOob / kAttnD;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        vraw[kt][r] = __builtin_amdgcn_raw_buffer_load_b128(vrs, (base + 16 * kt + 4 * o + r) * kAttnD + 16 * i, 0, kNt);
+      vsv[kt] = __builtin_amdgcn_raw_buffer_load_b128(vsr, (base + 16 * kt + 4 * o) * 4, 0, kNt);
+    }
+  };
+  fetch_k(b0 + wave);
+  fetch_v(b0 + wave);
+
+  // Q^T operand of MFMA (c, h): lane (i, o) holds row i of the tile, dims 64 c + 16 o + 8 h .. + 7. They sit
+  // in LDS in lane order: in registers they and O^T did not fit beside the block in flight.
+  char* const qs = (char*)lds + lane * 16;
+  size_t head[T];    // the lane's row as (token, query head)
+  uint32_t vis[T];   // the new keys it sees, bit r for row pos + r: i <= its token, or its tree ancestors
+  bool rvalid[T];
+  const int pl = a.parent && lane > 0 && lane < a.M ? attn_tree_parent(a.parent, lane) : 0;
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    const int row = 16 * (tile0 + t) + i;
+    rvalid[t] = row < rows;
+    const int qrow = rvalid[t] ? row : 0, qi = qrow / G;  // padding rows repeat row 0 and are not stored
+    head[t] = (size_t)qi * a.HQ + j * G + (qrow - qi * G);
+    u32x4a q[2];  // wave w brings c = w
+#pragma unroll
+    for (int h = 0; h < 2; ++h) q[h] = *(const u32x4a*)(a.q + head[t] * kAttnD + 64 * wave + 16 * o + 8 * h);
+#pragma unroll
+    for (int h = 0; h < 2; ++h) *(u32x4a*)(qs + ((t * 4 + wave) * 2 + h) * 1024) = q[h];
+    vis[t] = qi >= 31 ? ~0u : (2u << qi) - 1u;  // (no bit at or past M: qi < M)
+    if (a.parent) {
+      // the parents one per lane (one load for the wave), then the walk by shuffles
+      vis[t] = 1u;  // the root: every node sees it
+      int jn = qi;
+      for (int d = 0; d < kAttnMaxTree; ++d) {
+        vis[t] |= 1u << jn;
+        jn = __shfl(pl, jn);  // the root's entry is 0
+        if (__all(jn == 0)) break;
       }
-      st[kt] = c;
-    }
-    // mask, online softmax (this lane: one row, 8 keys), in log2 units: p = 2^(s - m) by
-    // v_exp_f32 (one instruction where expf takes a range reduction)
-    const float sl2 = a.scale * kLog2e;
-    float sc[8];
-    float mx = -INFINITY;
-    // a block of committed rows only (all before pos) needs no mask; in the others key rel =
-    // kidx - pos < M selects a bit of vis when >= 0
-    const bool committed = TREE && key0 + kAttnBlk <= pos;  // uniform
-    const int rel0 = TREE ? (int)(key0 - pos) + 4 * (lane >> 4) : 0;
-#pragma unroll
-    for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int rel = rel0 + 16 * kt + r;
-        const bool allowed =
-            TREE ? rvalid && (committed || (rel < a.M && (rel < 0 || ((vis >> rel) & 1u))))
-                 : rvalid && key0 + 16 * kt + 4 * (lane >> 4) + r < L && key0 + 16 * kt + 4 * (lane >> 4) + r <= qlimit;
-        const float v = allowed ? st[kt][r] * sl2 : -INFINITY;
-        sc[4 * kt + r] = v;
-        mx = fmaxf(mx, v);
-      }
-    mx = max_x32(max_x16(mx));
-    // Lazy rescale: the rows move to their new maxima (and O^T, l are scaled) only when some row
-    // of the wave gains more than kLazyMax (log2 units) over its running max; otherwise the block
-    // is summed against the running max, so p <= 2^kLazyMax. m, l and O^T stay consistent.
-    constexpr float kLazyMax = 8.f;
-    if (__ballot(mx > m_i + kLazyMax)) {  // uniform; a first finite maximum always counts
-      const float m_new = fmaxf(m_i, mx);
-      const float alpha = __builtin_amdgcn_exp2f(m_i - (m_new == -INFINITY ? 0.f : m_new));
-      m_i = m_new;
-      l_i *= alpha;
-#pragma unroll
-      for (int dt = 0; dt < 16; ++dt) acc[dt] = acc[dt] * alpha;
-    }
-    const float m_safe = m_i == -INFINITY ? 0.f : m_i;
-    float psum = 0.f;
-    uint32_t pb[4];
-#pragma unroll
-    for (int i = 0; i < 8; i += 2) {
-      const float p0 = __builtin_amdgcn_exp2f(sc[i] - m_safe), p1 = __builtin_amdgcn_exp2f(sc[i + 1] - m_safe);
-      psum += p0 + p1;
-      const int k0 = 16 * (i / 4) + 4 * (lane >> 4) + (i & 3);
-      pb[i / 2] = pk_bf16(p0 * vsc[k0], p1 * vsc[k0 + 1]);
-    }
-    psum = sum_x32(sum_x16(psum));
-    l_i += psum;
-    // O^T += V^T P^T: k-index 8 (l / 16) + i <-> key 4 (l / 16) + i (i < 4), 16 + 4 (l / 16) + i - 4
-    const bf16x8 pB = __builtin_bit_cast(bf16x8, make_uint4(pb[0], pb[1], pb[2], pb[3]));
-    const int vk = 4 * (lane >> 4);
-#pragma unroll
-    for (int dt = 0; dt < 16; ++dt) {
-      const uint16_t* vr = Vt + (16 * dt + (lane & 15)) * kVPitch;
-      const uint2 lo = *(const uint2*)(vr + vk), hi = *(const uint2*)(vr + 16 + vk);
-      acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, make_uint4(lo.x, lo.y, hi.x, hi.y)),
-                                                        pB, acc[dt], 0, 0, 0);
     }
   }
-  if (!computes || !rvalid) return;
-  // lanes with l / 16 == 0 .. 3 hold d = 16 dt + 4 (l / 16) + r of row l % 16
-  const size_t h = (size_t)qi * a.HQ + hq;
-  if (lane < 16) {
-    a.m_part[h * a.nsplit + s] = m_i;
-    a.l_part[h * a.nsplit + s] = l_i;
-  }
-  float* ap = a.acc_part + (h * a.nsplit + s) * kAttnD + 4 * (lane >> 4);
+  lds_barrier();
+
+  f32x4 acc[T][16];  // O^T tile e: dims 16 i' + e; lane (i, o), register r: row i, dim 64 o + 16 r + e
+  float m_i[T], l_i[T];
 #pragma unroll
-  for (int dt = 0; dt < 16; ++dt) *(float4*)(ap + 16 * dt) = make_float4(acc[dt][0], acc[dt][1], acc[dt][2], acc[dt][3]);
+  for (int t = 0; t < T; ++t) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[t][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+    m_i[t] = -INFINITY;
+    l_i[t] = 0.f;
+  }
+  const float sl2 = a.scale * kLog2e;
+  for (int blk = b0 + wave; blk < b1; blk += kAttnWaves) {
+    // S^T = K8 Q^T for the block's two 16-key tiles (fp8 is exact in bf16): lane (i, o) gets keys
+    // 16 kt + 4 o + r of row i; the key's scale multiplies the fp32 score
+    f32x4 st[T][2];
+#pragma unroll
+    for (int t = 0; t < T; ++t) st[t][0] = st[t][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const bf16x8 k0 = fp8x8_to_bf16(kraw[0][c][2 * h], kraw[0][c][2 * h + 1]);
+        const bf16x8 k1 = fp8x8_to_bf16(kraw[1][c][2 * h], kraw[1][c][2 * h + 1]);
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+          const bf16x8 q = *(const bf16x8*)(qs + ((t * 4 + c) * 2 + h) * 1024);
+          st[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, q, st[t][0], 0, 0, 0);
+          st[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, q, st[t][1], 0, 0, 0);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);  // bounds the operands made ahead
+    }
+    float kf[8], vf[8];
+#pragma unroll
+    for (int n = 0; n < 8; ++n) {
+      kf[n] = __uint_as_float(ksv[n / 4][n % 4]) * sl2;
+      vf[n] = __uint_as_float(vsv[n / 4][n % 4]);
+    }
+    fetch_k(blk + kAttnWaves);
+    const int64_t key0 = (int64_t)blk * kAttnBlk;
+    const bool committed = key0 + kAttnBlk <= pos;  // uniform: no new key in the block, nothing to mask
+    // online softmax in log2 units: p = 2^(s - m) by v_exp_f32
+    float sc[T][8];
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int n = 0; n < 8; ++n) sc[t][n] = st[t][n / 4][n % 4] * kf[n];
+    if (!committed) {
+      // bit 32 + r of a row's 64-bit word: key pos + r visible; committed keys (r < 0) always are. This lane's
+      // keys sit at bits 0-3 and 16-19 once the word is shifted to its first key.
+      const int sh = (int)(key0 - pos) + 4 * o + 32;  // 1 .. 75
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        const uint64_t word = ((uint64_t)vis[t] << 32) | 0xFFFFFFFFu;
+        const uint32_t seen = sh < 64 ? (uint32_t)(word >> (sh & 63)) : 0u;
+#pragma unroll
+        for (int n = 0; n < 8; ++n) sc[t][n] = (seen >> (16 * (n / 4) + n % 4)) & 1u ? sc[t][n] : -INFINITY;
+      }
+    }
+    // Rows keep the maximum of their first block as the reference m (p, l and O^T are floats: any common scale
+    // will do) until a key passes it by more than 2^kLazyMax. That key outweighs everything before it: 2^20
+    // keys at the old maximum are 2^-28 of it, below fp32's last bit, so the row's sums restart from zero.
+    // (Rescaling instead put O^T, which lives in AGPRs, through VGPRs and spilled.)
+    constexpr float kLazyMax = 48.f;
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      float mx = fmaxf(fmaxf(fmaxf(sc[t][0], sc[t][1]), fmaxf(sc[t][2], sc[t][3])),
+                       fmaxf(fmaxf(sc[t][4], sc[t][5]), fmaxf(sc[t][6], sc[t][7])));
+      mx = max_x32(max_x16(mx));
+      if (mx > m_i[t] + kLazyMax) {  // a first finite maximum always passes -inf
+        m_i[t] = mx;
+        l_i[t] = 0.f;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[t][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+    bf16x8 pb[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const float m_safe = m_i[t] == -INFINITY ? 0.f : m_i[t];
+      uint32_t w[4];
+#pragma unroll
+      for (int n = 0; n < 8; n += 2) {
+        const float p0 = __builtin_amdgcn_exp2f(sc[t][n] - m_safe), p1 = __builtin_amdgcn_exp2f(sc[t][n + 1] - m_safe);
+        l_i[t] += p0 + p1;  // this lane's keys; the octets' sums meet after the loop
+        w[n / 2] = pk_bf16(p0 * vf[n], p1 * vf[n + 1]);
+      }
+      pb[t] = __builtin_bit_cast(bf16x8, make_uint4(w[0], w[1], w[2], w[3]));
+    }
+    // O^T += V^T P^T: tile e takes byte e of the lane's eight keys (k-index 4 kt + r <-> key 16 kt + 4 o + r),
+    // one v_perm_b32 and one conversion (scale 1: exact) per pair
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+      const uint32_t sel = 0x0C0C0000u | ((4u + (e & 3)) << 8) | (uint32_t)(e & 3);  // byte 0 = second[e], byte 1 = first[e]
+      uint32_t w[4];
+#pragma unroll
+      for (int n = 0; n < 4; ++n) {
+        const uint32_t b = __builtin_amdgcn_perm(vraw[n / 2][2 * (n & 1) + 1][e / 4], vraw[n / 2][2 * (n & 1)][e / 4], sel);
+        w[n] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(b, 1.f, false));
+      }
+      const bf16x8 va = __builtin_bit_cast(bf16x8, make_uint4(w[0], w[1], w[2], w[3]));
+#pragma unroll
+      for (int t = 0; t < T; ++t) acc[t][e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pb[t], acc[t][e], 0, 0, 0);
+      if (e % 2) __builtin_amdgcn_sched_barrier(0);
+    }
+    fetch_v(blk + kAttnWaves);
+  }
+#pragma unroll
+  for (int t = 0; t < T; ++t) l_i[t] = sum_x32(sum_x16(l_i[t]));
+
+  // The waves meet in LDS, one query tile at a time: each puts its (m, l) and O^T there and
+  // sums its share of the O^T tiles over the waves, in wave order, at the common maximum.
+  constexpr int EP = 16 / kAttnWaves;
+  float* const ml = lds + (size_t)kAttnWaves * 4096;
+  float* const mine = lds + (size_t)wave * 4096 + lane * 4;
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    lds_barrier();  // the loop's Q reads, or the previous tile's, are done
+    if (o == 0) *(float2*)(ml + (wave * 16 + i) * 2) = make_float2(m_i[t], l_i[t]);
+#pragma unroll
+    for (int e = 0; e < 16; ++e) *(f32x4*)(mine + e * 256) = acc[t][e];
+    lds_barrier();
+    float2 p[kAttnWaves];
+    float m = -INFINITY, l = 0.f;
+#pragma unroll
+    for (int k = 0; k < kAttnWaves; ++k) {
+      p[k] = *(const float2*)(ml + (k * 16 + i) * 2);
+      m = fmaxf(m, p[k].x);
+    }
+    const float m_safe = m == -INFINITY ? 0.f : m;
+    f32x4 v[EP];
+#pragma unroll
+    for (int e = 0; e < EP; ++e) v[e] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < kAttnWaves; ++k) {
+      const float f = __builtin_amdgcn_exp2f(p[k].x - m_safe);
+      l += p[k].y * f;
+      const float* const from = lds + (size_t)k * 4096 + (EP * wave) * 256 + lane * 4;
+#pragma unroll
+      for (int e = 0; e < EP; ++e) v[e] = v[e] + *(const f32x4*)(from + e * 256) * f;
+    }
+    if (!rvalid[t]) continue;
+    float* const part = a.acc_part + (head[t] * a.nsplit + s) * kAttnD + 64 * o;
+    if (o == 0 && wave == 0) {
+      a.m_part[head[t] * a.nsplit + s] = m;
+      a.l_part[head[t] * a.nsplit + s] = l;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+      for (int e = 0; e < EP; e += 4)
+        *(float4*)(part + EP * wave + 16 * r + e) = make_float4(v[e][r], v[e + 1][r], v[e + 2][r], v[e + 3][r]);
+  }
 }
 
 // ------------------------------------------------------------------ reduce + output gate
@@ -446,8 +506,9 @@ struct AttnReduceArgs {
   const float* l_part;
   const float* acc_part;
   const uint16_t* qkv;  // [M, QKV] for the gates
+  const int64_t* pos;
   uint16_t* out;        // [M, HQ D]
-  int HQ, nsplit, ld;
+  int HQ, M, nsplit, ld;
 };
 
 // One workgroup of D threads per (token, query head). Every load is issued up front: the split
@@ -458,15 +519,15 @@ __global__ __launch_bounds__(kAttnD) void attn_reduce_kernel(AttnReduceArgs a) {
   constexpr int kB = 64;
   __shared__ float wsh[kMaxSplit], red[kAttnD / 64];
   const int h = blockIdx.x, d = threadIdx.x, lane = d & 63, wave = d >> 6;
-  const int ns = a.nsplit;
+  const int ns = AttnRange(*a.pos + a.M, a.nsplit).used(a.nsplit);  // the splits that hold keys
   const int t = h / a.HQ, hh = h % a.HQ;
   const uint16_t graw = a.qkv[(size_t)t * a.ld + (size_t)hh * 2 * kAttnD + kAttnD + d];
-  const float* ap = a.acc_part + (size_t)h * ns * kAttnD + d;
+  const float* ap = a.acc_part + (size_t)h * a.nsplit * kAttnD + d;
   float v[kB];
 #pragma unroll
   for (int i = 0; i < kB; ++i) v[i] = ap[(size_t)min(i, ns - 1) * kAttnD];
   const int sc = min(d, ns - 1);
-  const float m_s = a.m_part[(size_t)h * ns + sc], l_s = a.l_part[(size_t)h * ns + sc];
+  const float m_s = a.m_part[(size_t)h * a.nsplit + sc], l_s = a.l_part[(size_t)h * a.nsplit + sc];
   const bool mine = d < ns;  // ns <= kMaxSplit == kAttnD
   // maximum over the splits
   float mm = mine ? m_s : -INFINITY;
@@ -551,6 +612,26 @@ int attn_prep_launch(const void* qkv, int ld, const void* q_norm_w, const void* 
   return hipGetLastError() == hipSuccess ? TR_OK : TR_ERR_LAUNCH;
 }
 
+template <int T>
+hipError_t split_launch(const AttnSplitArgs& s, int wgs, int groups, hipStream_t stream) {
+  // the Q operands; after the loop each wave's O^T tile, then its (m, l) per row
+  constexpr size_t kLds = (size_t)kAttnWaves * (16384 + 16 * 8);
+  static_assert(T * 8192 <= kLds, "Q operands");
+  static std::atomic<uint64_t> raised{0};  // devices on which the kernel's LDS limit is raised
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) return e;
+  const uint64_t bit = 1ull << (dev & 63);
+  if (!(raised.load(std::memory_order_relaxed) & bit)) {
+    e = hipFuncSetAttribute(reinterpret_cast<const void*>(&attn_split_kernel<T>),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLds);
+    if (e != hipSuccess) return e;
+    raised.fetch_or(bit, std::memory_order_relaxed);
+  }
+  hipLaunchKernelGGL((attn_split_kernel<T>), dim3(wgs, groups), dim3(64 * kAttnWaves), kLds, stream, s);
+  return hipGetLastError();
+}
+
 int attn_decode_launch(const void* q, const void* qkv, int ld, const void* k_cache, const void* v_cache,
                        const float* k_scale, const float* v_scale, int maxlen, const int64_t* pos, void* out,
                        void* workspace, size_t workspace_bytes, int M, int HQ, int HKV, int D, int nsplit,
@@ -577,23 +658,27 @@ int attn_decode_launch(const void* q, const void* qkv, int ld, const void* k_cac
   s.maxlen = maxlen;
   s.nsplit = nsplit;
   s.scale = 1.f / sqrtf((float)D);
-  // the G M query rows of a kv head in groups of 64 (one 16-row tile per wave)
-  const int groups = ((HQ / HKV) * M + 16 * kAttnWaves - 1) / (16 * kAttnWaves);
-  if (parent)
-    hipLaunchKernelGGL(attn_split_kernel<true>, dim3(HKV * nsplit, groups), dim3(64 * kAttnWaves), 0,
-                       (hipStream_t)stream, s);
-  else
-    hipLaunchKernelGGL(attn_split_kernel<false>, dim3(HKV * nsplit, groups), dim3(64 * kAttnWaves), 0,
-                       (hipStream_t)stream, s);
-  if (hipGetLastError() != hipSuccess) return TR_ERR_LAUNCH;
+  // The G M query rows of a kv head in groups of up to three 16-row tiles, and as many key splits (nsplit at
+  // most) as leave one workgroup per CU: a CU holds one of them (see the kernel's registers), and every split
+  // costs its partials.
+  const int tiles = ((HQ / HKV) * M + 15) / 16, groups = (tiles + kAttnTiles - 1) / kAttnTiles;
+  const int fit = kAttnCUs / (HKV * groups);
+  s.nsplit = nsplit < fit ? nsplit : fit > 1 ? fit : 1;
+  const hipStream_t st = (hipStream_t)stream;
+  const int T = (tiles + groups - 1) / groups, wgs = HKV * s.nsplit;
+  const hipError_t e = T == 1 ? split_launch<1>(s, wgs, groups, st)
+                       : T == 2 ? split_launch<2>(s, wgs, groups, st) : split_launch<3>(s, wgs, groups, st);
+  if (e != hipSuccess) return TR_ERR_LAUNCH;
   AttnReduceArgs r;
   r.m_part = s.m_part;
   r.l_part = s.l_part;
   r.acc_part = s.acc_part;
   r.qkv = (const uint16_t*)qkv;
   r.out = (uint16_t*)out;
+  r.pos = pos;
   r.HQ = HQ;
-  r.nsplit = nsplit;
+  r.M = M;
+  r.nsplit = s.nsplit;
   r.ld = ld;
   hipLaunchKernelGGL(attn_reduce_kernel, dim3(M * HQ), dim3(kAttnD), 0, (hipStream_t)stream, r);
   return hipGetLastError() == hipSuccess ? TR_OK : TR_ERR_LAUNCH;

@@ -14,17 +14,16 @@ import torch
 
 from . import _lib
 
-NSPLIT = 64        # key-range splits of the flash-decoding kernel: 256 workgroups at 4 kv heads
-                   # (the reference uses 32 on a 170-SM part; measured fastest here)
+# Key-range splits of a flash-decoding call: what the workspace holds. The library takes this many or as many
+# as leave one workgroup per CU, whichever is less (64 at 4 kv heads, 16 for a 32-node tree at 24 / 4 heads).
+NSPLIT = 64
 CHAIN_NSPLIT = NSPLIT
-SPLIT_SLOTS = 512  # split-kernel workgroups resident at once: 256 CUs, two each (240 registers a lane)
+SPLIT_SLOTS = 512
 
 
 def tree_splits(M: int, cfg) -> int:
-    """Key-range splits for a draft tree of M nodes: its G M query rows per kv head run in groups of
-    64 (a second grid dimension), so the grid is HKV x splits x groups; the largest count up to
-    NSPLIT whose grid fits one pass of SPLIT_SLOTS (42 for 32 nodes at 24 / 4 heads: 21% faster
-    per call than 64, which needs a second pass)."""
+    """Key-range splits a draft tree of M nodes sizes its workspace for: the largest count up to NSPLIT with
+    HKV x splits x (groups of 64 query rows) within SPLIT_SLOTS (42 for 32 nodes at 24 / 4 heads)."""
     groups = -(-(cfg.n_heads // cfg.n_kv_heads) * M // 64)
     return max(1, min(NSPLIT, SPLIT_SLOTS // (cfg.n_kv_heads * groups)))
 
