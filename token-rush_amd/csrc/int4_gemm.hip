@@ -203,6 +203,12 @@ __device__ __forceinline__ int udiv_small(uint32_t q, int d, uint32_t magic) {
   return d == 1 ? (int)q : (int)__umulhi(q, magic);
 }
 
+}  // namespace tr
+
+#include "rows32_gemm.h"
+
+namespace tr {
+
 // One accumulator tile element: (mt, lane, r) -> output row m = 16 mt + 4 (lane / 16) + r,
 // column n = 16 strip + lane % 16.
 template <int MT, int GW, bool F16S, bool XSTAGE>
@@ -712,6 +718,37 @@ hipError_t launch_t(GemmArgs a, const Plan& p, hipStream_t stream) {
   return hipGetLastError();
 }
 
+// rows32_gemm_kernel (the measurements beside it): one K slot, R_req strips per workgroup (<= 0: one workgroup per CU).
+bool wide_shape(int M, int K) { return M > 16 && K / kGroup > 24 && K / kGroup <= 5 * kWideWaves; }
+
+template <int GW, bool F16S>
+hipError_t launch_wide(GemmArgs a, int R_req, hipStream_t stream) {
+  static bool raised = false;
+  if (!raised) {
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&rows32_gemm_kernel<GW, F16S>),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsMax);
+    if (e != hipSuccess) return e;
+    raised = true;
+  }
+  const int nstrips = a.N / 16, W = (a.K / kGroup + GW - 1) / GW;
+  a.R = R_req <= 0 ? (nstrips + kCUs - 1) / kCUs : R_req < nstrips ? R_req : nstrips;
+  a.gn = (nstrips + a.R - 1) / a.R;
+  a.rfull = nstrips - (a.R - 1) * a.gn;
+  const size_t per_strip = (size_t)W * 2 * 256 * sizeof(float);
+  const int rb = (int)(kLdsMax / (2 * per_strip));
+  a.RB = rb > 4 ? 4 : rb;
+  const size_t ring = 2 * a.RB * per_strip, stage = (size_t)W * 8192;
+  hipLaunchKernelGGL((rows32_gemm_kernel<GW, F16S>), dim3(a.gn), dim3(64 * W), ring > stage ? ring : stage, stream, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_wide_gw(const GemmArgs& a, int R_req, int scale_dtype, hipStream_t stream) {
+  const bool f16 = scale_dtype == 1;
+  if (a.K / kGroup <= 4 * kWideWaves)
+    return f16 ? launch_wide<4, true>(a, R_req, stream) : launch_wide<4, false>(a, R_req, stream);
+  return f16 ? launch_wide<5, true>(a, R_req, stream) : launch_wide<5, false>(a, R_req, stream);
+}
+
 hipError_t launch(const GemmArgs& a, const Plan& p, int scale_dtype, hipStream_t stream) {  // NOLINT
   const bool f16 = scale_dtype == 1;
   if (a.M > 16) return f16 ? launch_t<2, 2, true, true>(a, p, stream) : launch_t<2, 2, false, true>(a, p, stream);
@@ -817,6 +854,11 @@ static int gemm_impl(const void* x, const void* packed, void* out, void* partial
     const size_t need = ws_counter_bytes() + (size_t)p.S * M * N * sizeof(float);
     if (!workspace || workspace_bytes < need) return TR_ERR_ARG;
     if (p.grid_n > kWsCounters) return TR_ERR_CONFIG;
+    if (wide_shape(M, K) && n_slots <= 0) {  // default slots: one after all, and no partials
+      a.mode = OUT_BF16;
+      a.out = out;
+      return launch_wide_gw(a, R, scale_dtype, (hipStream_t)stream) == hipSuccess ? TR_OK : TR_ERR_LAUNCH;
+    }
     if (silu) {
       // the K slots' partials into the workspace, then their sum and silu in a second launch
       float* part = (float*)((char*)workspace + ws_counter_bytes());
