@@ -24,6 +24,7 @@
 // Work split ("activation-stationary"): a workgroup owns every grid_n-th strip and a K slot; each
 // of its W waves owns one K block of GW groups (GW = 4 for M <= 16, 2 above), loads that
 // block's activations into registers once, then streams the strips' tiles for its block.
+// M > 16 in out mode takes rows32_gemm.h's kernel at 24 < K / 128 <= 40.
 // After every few strips the waves' partial tiles are summed through LDS in fixed wave order
 // (deterministic). With S > 1 slots, slots write fp32 partials: either the caller's
 // [S, M, N] buffer (the contract of the reference's partials(), tokenrush/quant.py:381-391,
@@ -37,7 +38,7 @@ namespace tr {
 
 // In-kernel timeline (a build with -DTR_TIMELINE only, `make timeline`): wave w of workgroup b
 // writes s_memrealtime (100 MHz) at mark i to tr_tl_buf[(b * 16 + w) * kTlMarks + i]. Marks: 0
-// entry, 1 launch constants ready, 2 activations staged, 3 the first two strips issued, 4
+// entry, 1 launch constants ready, 2 activations staged, 3 the first strips issued, 4
 // prologue end (group sums), 5 + r strip r's MACs done (r < 11), 16 a batch's reduction done,
 // 20 exit of the strip loop, 21 the activation loads issued, 22 past the barrier that orders
 // them before the strips. The normal build has none of it.
@@ -78,24 +79,31 @@ struct Strip {
 // parameters are loaded first: every group's fold needs them, so vmcnt then lets the first
 // group start as soon as its own codes arrive.
 template <int GW>
-__device__ __forceinline__ void load_strip(Strip<GW>& t, __amdgpu_buffer_rsrc_t rsrc, int soff, int lane_off,
-                                           int sm_voff) {
-  if (GW == 4) {
+__device__ __forceinline__ void load_params(uint32_t (&sm)[GW], __amdgpu_buffer_rsrc_t rsrc, int soff, int sm_voff) {
+  if constexpr (GW == 4) {
     const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, sm_voff, soff, 2 /* nt */);
-    t.sm[0] = v.x;
-    t.sm[1] = v.y;
-    t.sm[2 % GW] = v.z;
-    t.sm[3 % GW] = v.w;
+    sm[0] = v.x;
+    sm[1] = v.y;
+    sm[2] = v.z;
+    sm[3] = v.w;
   } else {
     const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(rsrc, sm_voff, soff, 2 /* nt */);
-    t.sm[0] = v.x;
-    t.sm[1] = v.y;
+    sm[0] = v.x;
+    sm[1] = v.y;
   }
+}
+
+__device__ __forceinline__ uint4 load_codes(__amdgpu_buffer_rsrc_t rsrc, int soff, int off) {
+  const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, soff, 2 /* nt */);
+  return make_uint4(v.x, v.y, v.z, v.w);
+}
+
+template <int GW>
+__device__ __forceinline__ void load_strip(Strip<GW>& t, __amdgpu_buffer_rsrc_t rsrc, int soff, int lane_off,
+                                           int sm_voff) {
+  load_params<GW>(t.sm, rsrc, soff, sm_voff);
 #pragma unroll
-  for (int gw = 0; gw < GW; ++gw) {
-    const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(rsrc, lane_off + gw * kCodeBytes, soff, 2 /* nt */);
-    t.w[gw] = make_uint4(v.x, v.y, v.z, v.w);
-  }
+  for (int gw = 0; gw < GW; ++gw) t.w[gw] = load_codes(rsrc, soff, lane_off + gw * kCodeBytes);
 }
 
 // E = sum over the group of x * (128 + q), then acc += s * E. The group's other term,
@@ -195,7 +203,7 @@ struct GemmArgs {
   int* am_cnt;            // arrival counter, zero between calls
   const int64_t* spec;    // [M] committed token + drafts, or null (argmax only)
   AcceptOut o;            // o.pred [M] always; the rest when spec != null
-  int xstage_off;         // byte offset of the activation staging area in dynamic LDS (M <= 8, M > 16)
+  int xstage_off;         // byte offset of the activation staging area in dynamic LDS
 };
 
 // q / d for q < 2^16 and 1 <= d < 2^15, magic = ceil(2^32 / d) (d == 1 has no 32-bit magic).
@@ -210,9 +218,24 @@ __device__ __forceinline__ int udiv_small(uint32_t q, int d, uint32_t magic) {
 namespace tr {
 
 // One accumulator tile element: (mt, lane, r) -> output row m = 16 mt + 4 (lane / 16) + r,
-// column n = 16 strip + lane % 16.
-template <int MT, int GW, bool F16S, bool XSTAGE>
+// column n = 16 strip + lane % 16. XR = 8, 16 or 32: the most rows of x, staged in one pass of 8,
+// two of 8, or two of 16.
+//
+// Strips in flight. At one row tile a wave holds one strip, and each group's codes are reloaded for
+// the next strip as soon as the group is dequantized, so a group waits for its own load only and
+// the loads spread over the strip's MACs. Two strips in flight, each refilled after its last MAC,
+// sent the refill out in one burst with nothing to cover it but the other strip. Bound as before by
+// the instructions and waits of a strip (at 34816 x 5120 the codes and parameters alone take 18 us
+// at 5.1 TB/s, so that shape is now at memory speed). us, graph of launches, two strips -> one:
+//   M = 1: 5120 x 5120 6.3 -> 5.4, 7168 x 5120 7.0 -> 6.1, 14336 x 5120 10.3 -> 9.3, 16384 x 5120
+//     11.5 -> 10.2, gate/up 34816 x 5120 19.5 -> 18.4, 5120 x 6144 partials 6.0 -> 5.5, 8192 x 2048
+//     4.7 -> 4.5; 5120 x 17408 partials 10.6 / 10.7 and 248320 x 5120 108 / 108 (memory).
+//   M = 8: 7.0 -> 6.3, 7.5 -> 6.5, 10.8 -> 10.0, 11.7 -> 10.6, 20.2 -> 18.7, 6.2 -> 6.0, 5.0 -> 4.7.
+// At two row tiles two strips stay: a group's MACs are twice as long and there are two groups to
+// a wave (M = 32 partials of 5120 x 6144 9.1 with two, 10.0 with one; 5120 x 17408 17.5 / 18.5).
+template <int XR, bool F16S>
 __global__ __launch_bounds__(768) void int4_gemm_kernel(GemmArgs a) {
+  constexpr int MT = XR > 16 ? 2 : 1, GW = MT == 1 ? 4 : 2, kInFlight = MT;
   // 16-byte aligned: the dynamic area follows the kernel's 776 bytes of static LDS, and the
   // ring's and staging area's 16-byte accesses stall when misaligned (SQ_LDS_UNALIGNED_STALL)
   extern __shared__ __attribute__((aligned(16))) float red[];  // [2][RB][W][MT][64][4]
@@ -259,34 +282,37 @@ __global__ __launch_bounds__(768) void int4_gemm_kernel(GemmArgs a) {
   // A-operand layout (lane l: row l % 16 of its row tile, k = 32 j + 8 (l / 16) .. + 7 of MFMA j).
   // Padding groups (g >= G) read group G - 1: finite values that meet zero scale and min.
   uint4 xa[GW][MT][4];
-  constexpr int kXL = MT == 1 ? 8 : 16;  // staging loads per wave: one per row (GW = 4), or per row pair (GW = 2)
+  constexpr int kXL = XR == 8 ? 8 : 16;  // staging loads per wave: one per row (GW = 4), or per row pair (GW = 2)
   uint4 xv[kXL];                         // staged rows, held in VGPRs until they are written to LDS
-  if constexpr (XSTAGE) {
-    // M <= 8: load the rows coalesced into VGPRs, write them to this wave's LDS staging area,
+  {
+    // M <= 16: load the rows coalesced into VGPRs, write them to this wave's LDS staging area,
     // then read them back in the operand layout. In the operand layout itself consecutive lanes
     // would read different rows, each lane a separate cache access, which took 3-6 us for these
     // 8 KB per wave. Loading straight into LDS (buffer_load ... lds) lands no earlier and made the
     // M = 8 layer set 0.8 us slower than this register round trip. Load t brings row t of the wave's four
-    // groups (lane l: group l / 16, 16-byte chunk (l % 16) ^ t), so a call issues M loads, one per
+    // groups (lane l: group l / 16, 16-byte chunk (l % 16) ^ (t % 8)), so a call issues M loads, one per
     // real row: every load instruction costs the CU's address unit the same 16 cycles whether
-    // its lanes fetch or not. The staging area holds row r of group gw at (r GW + gw) 256 bytes,
-    // chunk k of the row in 16-byte slot k ^ r, so the 16 rows read by one operand load fall in
-    // different LDS banks.
+    // its lanes fetch or not. The staging area holds row r of group gw at (r % 8 GW + gw) 256 bytes,
+    // chunk k of the row in 16-byte slot k ^ r % 8, so the rows read by one operand load fall in
+    // different LDS banks. Rows 8 to 15 follow rows 0 to 7 through the same 8 KB per wave. Lanes
+    // past row M - 1 take that row; their outputs are never stored. M = 9..16 loaded the operand
+    // layout directly before: M = 16 us, before -> now with one strip in flight, 5120 x 5120
+    // 9.4 -> 7.6, 7168 x 5120 9.8 -> 7.8, 16384 x 5120 14.2 -> 12.1, gate/up 22.4 -> 20.5,
+    // 5120 x 6144 partials 8.4 -> 7.3, 5120 x 17408 15.0 -> 12.5, 8192 x 2048 7.2 -> 5.7.
     //
     // M = 17..32 (two row tiles, two groups per wave): load u brings rows 2u and 2u + 1 (lanes
     // 0-31 and 32-63; lane l: group (l / 16) % 2, chunk (l % 16) ^ (row % 16)), all 16 loads
     // issued before the strips, and the 16-row tiles are staged one after the other through the
     // same 8 KB per wave. That area lies inside the reduction ring, which is first written after
     // the prologue (an LDS barrier orders them). Rows >= M load from beyond the resource: zeros.
-    static_assert((MT == 1 && GW == 4) || (MT == 2 && GW == 2), "activation staging: 1 x 4 or 2 x 2 tiles");
     const auto xrs = __builtin_amdgcn_make_buffer_rsrc((void*)a.x, (short)0, a.M * a.K * 2, 0x00020000);
     const int lk = lane & 15;
     if constexpr (MT == 1) {
       const int g = min(gbase + (lane >> 4), G - 1);
 #pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        if (t >= a.M) break;
-        const int off = (t * a.K + g * kGroup) * 2 + ((lk ^ t) & 15) * 16;
+      for (int t = 0; t < XR; ++t) {
+        if (t >= a.M) continue;
+        const int off = (t * a.K + g * kGroup) * 2 + (lk ^ (t & 7)) * 16;
         const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 0, 0);
         xv[t] = make_uint4(v.x, v.y, v.z, v.w);
       }
@@ -300,61 +326,58 @@ __global__ __launch_bounds__(768) void int4_gemm_kernel(GemmArgs a) {
         xv[u] = make_uint4(v.x, v.y, v.z, v.w);
       }
     }
-  } else {
-#pragma unroll
-    for (int gw = 0; gw < GW; ++gw) {
-      const int g = min(gbase + gw, G - 1);
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const int xr = min(16 * mt + (lane & 15), a.M - 1);
-        const uint4* p = (const uint4*)(a.x + (size_t)xr * a.K + g * kGroup + 8 * (lane >> 4));
-#pragma unroll
-        for (int j = 0; j < 4; ++j) xa[gw][mt][j] = p[4 * j];  // k = 32 j + 8 (lane / 16) .. + 7
-      }
-    }
   }
-  // Two strips in flight, issued after the activation loads (vmcnt counts loads in issue order,
+  // The first strips, issued after the activation loads (vmcnt counts loads in issue order,
   // so waiting for the activations leaves the strips in flight). Waves without a K block issue
   // out-of-range loads: no memory access, the same count.
-  Strip<GW> buf[2];
-  // Staged kernels: every wave's activation requests enter the CU's in-order memory pipeline
-  // before any wave's weight requests, so no wave waits for its activations behind the other
-  // waves' strips.
+  Strip<GW> buf[kInFlight];
+  // Every wave's activation requests enter the CU's in-order memory pipeline before any wave's
+  // weight requests, so no wave waits for its activations behind the other waves' strips.
   TLM(21);
-  if constexpr (XSTAGE) __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_s_barrier();
   TLM(22);
-  load_strip<GW>(buf[0], rsrc, active ? strip_off(r0) : oob, lane_off, sm_voff);
-  load_strip<GW>(buf[1], rsrc, active ? strip_off(r0 + 1) : oob, lane_off, sm_voff);
-  TLM(3);
-  if constexpr (XSTAGE) {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * (GW + 1)) : "memory");  // the staging loads have landed
-    TLM(2);
-    char* stage = (char*)red + a.xstage_off + wave * (GW * 256 * (MT == 1 ? 8 : 16));
-    const int i = lane & 15;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      if constexpr (MT == 1) {
+  for (int h = 0; h < kInFlight; ++h) load_strip<GW>(buf[h], rsrc, active ? strip_off(r0 + h) : oob, lane_off, sm_voff);
+  TLM(3);
+  {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kInFlight * (GW + 1)) : "memory");  // the staging loads have landed
+    TLM(2);
+    char* stage = (char*)red + a.xstage_off + wave * 8192;
+    const int i = lane & 15;
+    if constexpr (MT == 1) {
+#pragma unroll
+      for (int p = 0; p < XR / 8; ++p) {
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
-          if (t >= a.M) break;
-          *(uint4*)(stage + t * 1024 + lane * 16) = xv[t];  // lane l: chunk l % 16 of group l / 16
+          if (8 * p + t >= a.M) continue;
+          *(uint4*)(stage + t * 1024 + lane * 16) = xv[8 * p + t];  // lane l: chunk l % 16 of group l / 16
         }
-      } else {
+        const int rs = p ? min(i, a.M - 1) - 8 : min(min(i, 7), a.M - 1);  // staged row
+        if (p == 0 || i >= 8) {
+#pragma unroll
+          for (int gw = 0; gw < GW; ++gw)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+              xa[gw][0][j] = *(const uint4*)(stage + (rs * GW + gw) * 256 + ((4 * j + (lane >> 4)) ^ rs) * 16);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
 #pragma unroll
         for (int u = 0; u < 8; ++u) *(uint4*)(stage + u * 1024 + lane * 16) = xv[8 * mt + u];  // rows 2u, 2u + 1
-      }
 #pragma unroll
-      for (int gw = 0; gw < GW; ++gw) {
+        for (int gw = 0; gw < GW; ++gw) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const int k = 4 * j + (lane >> 4);
-          const int rs = MT == 1 ? (i & 7) : i;  // staged row
-          const uint4 v = *(const uint4*)(stage + (rs * GW + gw) * 256 + ((k ^ i) & 15) * 16);
-          xa[gw][mt][j] = 16 * mt + i < a.M ? v : make_uint4(0u, 0u, 0u, 0u);
+          for (int j = 0; j < 4; ++j) {
+            const int k = 4 * j + (lane >> 4);
+            const uint4 v = *(const uint4*)(stage + (i * GW + gw) * 256 + ((k ^ i) & 15) * 16);
+            xa[gw][mt][j] = 16 * mt + i < a.M ? v : make_uint4(0u, 0u, 0u, 0u);
+          }
         }
       }
+      lds_barrier();  // every wave's staging reads before any ring write
     }
-    if constexpr (MT == 2) lds_barrier();  // every wave's staging reads before any ring write
   }
 
   // Xa[mt] = sum of x over group gbase + lane / 16 for row 16 mt + lane % 16 (the A operand of
@@ -392,14 +415,27 @@ __global__ __launch_bounds__(768) void int4_gemm_kernel(GemmArgs a) {
   // batch's writes never race the previous batch's reads.
   const int RB = a.RB;
   int sib = 0, half = 0;  // position in the current batch, ring half (wave-uniform)
-  for (int rb = r0; rb < r1; rb += 2) {
+  for (int rb = r0; rb < r1; rb += kInFlight) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
+    for (int h = 0; h < kInFlight; ++h) {
       const int r = rb + h;
       f32x4 acc[MT];
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) acc[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (active && r < r1) {
+      if constexpr (kInFlight == 1) {
+        // Waves without a K block compute on zeros, so that every path issues the refill.
+        const int next = active ? strip_off(r + 1) : oob;
+        uint32_t sm[GW];
+#pragma unroll
+        for (int gw = 0; gw < GW; ++gw) {
+          tile_mac<MT, F16S>(buf[h].w[gw], buf[h].sm[gw], xa[gw], acc, kExp128);
+          if (gw == 0) load_params<GW>(sm, rsrc, next, sm_voff);
+          buf[h].w[gw] = load_codes(rsrc, next, lane_off + gw * kCodeBytes);
+        }
+        min_fold<MT, GW, F16S>(buf[h].sm, Xa, slot16, acc);
+#pragma unroll
+        for (int gw = 0; gw < GW; ++gw) buf[h].sm[gw] = sm[gw];
+      } else if (active && r < r1) {
 #pragma unroll
         for (int gw = 0; gw < GW; ++gw) tile_mac<MT, F16S>(buf[h].w[gw], buf[h].sm[gw], xa[gw], acc, kExp128);
         min_fold<MT, GW, F16S>(buf[h].sm, Xa, slot16, acc);
@@ -414,7 +450,7 @@ __global__ __launch_bounds__(768) void int4_gemm_kernel(GemmArgs a) {
       // range: zeros, no memory access), so every path has the same loads in flight and the
       // compiler's wait before the next strip's compute covers that strip's loads only -- a
       // refill under a branch made it wait for the other buffer's loads as well.
-      load_strip<GW>(buf[h], rsrc, active ? strip_off(r + 2) : oob, lane_off, sm_voff);
+      if constexpr (kInFlight == 2) load_strip<GW>(buf[h], rsrc, active ? strip_off(r + 2) : oob, lane_off, sm_voff);
       if (r < r1) {
         float* ring = red + (size_t)half * RB * W * MT * 256;
         if (active) {
@@ -578,9 +614,10 @@ __global__ __launch_bounds__(768) void int4_gemm_kernel(GemmArgs a) {
 // The gate/up pair layout with more than one K slot: the slots' fp32 partials [S, M, N] summed in
 // slot order, four outputs per thread; output (m, 8 s + j) is silu(bf16(g)) * bf16(u) with g, u
 // the sums of columns 16 s + j and 16 s + 8 + j (the epilogue's arithmetic). A second launch
-// instead of the GEMM's last-arriver sum: that tail loads two partials per output, and at M = 32
-// gate_up took 37.2-37.6 us with it against 35.0 us for partials plus this kernel. Plain out mode
-// keeps the in-kernel sum (qkv 12.8-13.1 us with it, 13.1-14.3 us with a second launch).
+// instead of the GEMM's last-arriver sum: that tail loads two partials per output (34816 x 5120 at
+// two slots and M = 32: 37.2-37.6 us with it against 35.0 us for partials plus this kernel). Plain
+// out mode keeps the in-kernel sum (7168 x 5120 12.8-13.1 us with it, 13.1-14.3 us with a second
+// launch). Reached where one slot does not hold K: K > 6144, at M > 16 K > 5120, or explicit slots.
 __global__ __launch_bounds__(256) void slot_sum_kernel(const float* __restrict__ part, int S, int M, int N,
                                                        uint16_t* __restrict__ out) {
   const size_t slot = (size_t)M * N;
@@ -633,13 +670,15 @@ bool make_plan(int N, int K, int M, int S_req, int R_req, Plan* p);
 
 // The partial-mode plan (the caller sums the slots, so more K slots cost only their writes, not
 // a last-arriver slot sum): the slot count from the default's up to 6 with the least work on the
-// busiest CU, rounds of workgroups x strips x waves, the smaller count on ties. The staged M <= 8
+// busiest CU, rounds of workgroups x strips x waves, the smaller count on ties. The M <= 8
 // kernel also counts its prologue (activation staging and group sums, ending ~4.7 us after launch
 // against ~1.2 us per strip) as kRampStrips strips per workgroup, which favours fewer waves per
 // workgroup. Measured at M = 8 (graph of launches, us): the 5120 x 6144 projection 7.31 at 1
 // slot, 9.55 at 2, 6.54 at the chosen 3, 7.43 at 4; 5120 x 17408 12.35 at 3, 11.93 at 4, 11.67
-// at the chosen 5, 13.96 at 6 (M = 1: 11.6, 11.7, 10.47, 12.3). At M = 16 (unstaged) 5120 x 17408
-// ran 14.13 at 4 and 14.35 at 5 slots, and keeps 4.
+// at the chosen 5, 13.96 at 6 (M = 1: 11.6, 11.7, 10.47, 12.3). At M = 16 5120 x 17408
+// ran 14.13 at 4 and 14.35 at 5 slots, and keeps 4. These are the counts that callers see, measured
+// with two strips in flight; with one, 3 slots lead for 5120 x 17408 too (M = 8 10.7 us at 3, 11.2 at
+// 4, 11.5 at 5; M = 16 12.5, 13.1, 14.0) and 5120 x 6144 keeps 3 (6.2; 7.2 at 4).
 constexpr long kRampStrips = 3;
 bool make_partial_plan(int N, int K, int M, Plan* p) {
   Plan best;
@@ -686,20 +725,20 @@ bool make_plan(int N, int K, int M, int S_req, int R_req, Plan* p) {
   return true;
 }
 
-template <int MT, int GW, bool F16S, bool XSTAGE>
+template <int XR, bool F16S>
 hipError_t launch_t(GemmArgs a, const Plan& p, hipStream_t stream) {
+  constexpr int MT = XR > 16 ? 2 : 1;
   const dim3 grid(p.grid_n * p.S), block(64 * p.W);
   const size_t per_strip = (size_t)p.W * MT * 256 * sizeof(float);
-  // Ring budget: the staged kernel keeps 64 KB (its staging takes the rest); the others share
-  // the CU's LDS among the workgroups the plan puts on one CU, so larger batches never cost
-  // occupancy.
-  // The two-tile staging area shares the ring (it is dead before the first partial is written).
-  constexpr bool kShared = XSTAGE && MT == 2;
+  // Ring budget: at one row tile 64 KB (the staging area takes the rest). The two-tile staging
+  // area shares the ring (it is dead before the first partial is written), which shares the CU's
+  // LDS among the workgroups the plan puts on one CU, so larger batches never cost occupancy.
+  constexpr bool kShared = MT == 2;
   const int wg_per_cu = p.W >= kWavesPerCU ? 1 : kWavesPerCU / p.W;
-  int rb = (int)(((XSTAGE && !kShared) ? kLdsBudget : kLdsMax / wg_per_cu) / (2 * per_strip));
+  int rb = (int)((!kShared ? kLdsBudget : kLdsMax / wg_per_cu) / (2 * per_strip));
   a.RB = rb < 1 ? 1 : (rb > 4 ? 4 : rb);
   const size_t ring = 2 * a.RB * per_strip;
-  const size_t stage = XSTAGE ? (size_t)p.W * GW * 256 * (MT == 1 ? 8 : 16) : 0;
+  const size_t stage = (size_t)p.W * 8192;
   a.xstage_off = kShared ? 0 : (int)ring;
   const size_t lds = kShared ? (ring > stage ? ring : stage) : ring + stage;
   {
@@ -707,14 +746,14 @@ hipError_t launch_t(GemmArgs a, const Plan& p, hipStream_t stream) {
     // kernel's limit once
     static bool raised = false;
     if (!raised) {
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&int4_gemm_kernel<MT, GW, F16S, XSTAGE>),
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&int4_gemm_kernel<XR, F16S>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsMax);
       if (e != hipSuccess) return e;
       raised = true;
     }
     if (lds > kLdsMax) return hipErrorInvalidValue;
   }
-  hipLaunchKernelGGL((int4_gemm_kernel<MT, GW, F16S, XSTAGE>), grid, block, lds, stream, a);
+  hipLaunchKernelGGL((int4_gemm_kernel<XR, F16S>), grid, block, lds, stream, a);
   return hipGetLastError();
 }
 
@@ -751,9 +790,9 @@ hipError_t launch_wide_gw(const GemmArgs& a, int R_req, int scale_dtype, hipStre
 
 hipError_t launch(const GemmArgs& a, const Plan& p, int scale_dtype, hipStream_t stream) {  // NOLINT
   const bool f16 = scale_dtype == 1;
-  if (a.M > 16) return f16 ? launch_t<2, 2, true, true>(a, p, stream) : launch_t<2, 2, false, true>(a, p, stream);
-  if (a.M <= 8) return f16 ? launch_t<1, 4, true, true>(a, p, stream) : launch_t<1, 4, false, true>(a, p, stream);
-  return f16 ? launch_t<1, 4, true, false>(a, p, stream) : launch_t<1, 4, false, false>(a, p, stream);
+  if (a.M > 16) return f16 ? launch_t<32, true>(a, p, stream) : launch_t<32, false>(a, p, stream);
+  if (a.M <= 8) return f16 ? launch_t<8, true>(a, p, stream) : launch_t<8, false>(a, p, stream);
+  return f16 ? launch_t<16, true>(a, p, stream) : launch_t<16, false>(a, p, stream);
 }
 
 }  // namespace
