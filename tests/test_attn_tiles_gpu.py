@@ -81,3 +81,11 @@ def test_split_counts(dev, nsplit, tree):
 def test_growing_scores(dev, nsplit):
     run(dev, 8, 6, 1, 1500, False, nsplit, spikes=True)
     run(dev, 20, 6, 1, 700, True, nsplit, spikes=True)
+
+
+@pytest.mark.parametrize("M", [1, 5, 8])
+@pytest.mark.parametrize("pos", [503, 504, 511, 512, 1016, 1023, 1024, 1030])
+@pytest.mark.parametrize("spikes", [False, True])
+def test_rounds_per_split(dev, M, pos, spikes):
+    """Four splits of one, two and three rounds of four blocks, one to three query tiles."""
+    run(dev, M, 6, 1, pos, False, 4, seed=pos, spikes=spikes)

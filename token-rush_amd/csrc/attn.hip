@@ -25,7 +25,14 @@
 //   eight is the A operand of O^T tile e (dims 16 i + e), so V is transposed in registers, by v_perm_b32.
 //   Row maxima need two permlane swaps, row sums are made after the loop. After the last block the waves'
 //   (m, l, O^T) meet in LDS.
-// Each wave keeps O^T for up to 48 rows x 256 d in 192 AGPRs, one workgroup per CU, so the launch takes as
+// A split of one or two rounds of four blocks does not merge O^T: the waves' P^T meet in LDS instead, and each
+// wave makes a quarter of the dims over all of a round's blocks (attn_split_kernel's `shared`). The merge of
+// three tiles was 3 of 9 us there; with the last round's empty prefetches gone and O^T transposed over the octets,
+// so that its stores are 64 contiguous bytes a row, split + combine over 1k rows went, us: 1 token 9.5 -> 8.5,
+// 8 tokens 15.0 -> 12.9, a 32-node tree 20.5 -> 17.8. What is left of the split at 8 tokens over 8100 rows (9.1 us
+// from entry): 4.4 until K, V and Q are there (17 MB), 2.7 for scores, probabilities and O^T, 1.9 for 12.6 MB of
+// partials.
+// Each wave otherwise keeps O^T for up to 48 rows x 256 d in 192 AGPRs, one workgroup per CU, so the launch takes as
 // many splits as leave one workgroup per CU.
 //
 // Before, four waves converted each block into LDS together (two barriers and a transposed write per block)
@@ -98,6 +105,21 @@ __device__ __forceinline__ float max_x16(float v) {
 __device__ __forceinline__ float max_x32(float v) {
   const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+
+// Lane (i, o) with elements r -> lane (i, r) with elements o: four by four over a wave's rows of 16 lanes.
+__device__ __forceinline__ f32x4 transpose_octets(f32x4 v) {
+  uint32_t x[4];
+#pragma unroll
+  for (int n = 0; n < 4; ++n) {
+    const float f = v[n];
+    x[n] = __float_as_uint(f);
+  }
+  const auto a = __builtin_amdgcn_permlane16_swap(x[0], x[1], false, false);
+  const auto b = __builtin_amdgcn_permlane16_swap(x[2], x[3], false, false);
+  const auto c = __builtin_amdgcn_permlane32_swap(a[0], b[0], false, false);
+  const auto d = __builtin_amdgcn_permlane32_swap(a[1], b[1], false, false);
+  return f32x4{__uint_as_float(c[0]), __uint_as_float(d[0]), __uint_as_float(c[1]), __uint_as_float(d[1])};
 }
 
 // ------------------------------------------------------------------ prep
@@ -310,8 +332,35 @@ __global__ __launch_bounds__(64 * kAttnWaves, 1) void attn_split_kernel(AttnSpli
       vsv[kt] = __builtin_amdgcn_raw_buffer_load_b128(vsr, (base + 16 * kt + 4 * o) * 4, 0, kNt);
     }
   };
+  // A round of the short ranges: the wave's quarter of the dims of the round's four blocks (lane (i, o): dims
+  // 64 wave + 4 i .. + 3 of keys 16 kt + 4 o + r), and the scales of its own block
+  uint32_t vq[kAttnWaves][8];
+  auto fetch_vq = [&](int blk0) {
+#pragma unroll
+    for (int b = 0; b < kAttnWaves; ++b) {
+      const uint32_t base = blk0 + b < b1 ? (uint32_t)(blk0 + b) * kAttnBlk : kOob / kAttnD;
+#pragma unroll
+      for (int n = 0; n < 8; ++n)
+        vq[b][n] = __builtin_amdgcn_raw_buffer_load_b32(vrs, (base + 16 * (n / 4) + 4 * o + n % 4) * kAttnD + 64 * wave + 4 * i,
+                                                        0, kNt);
+    }
+  };
+  auto fetch_vs = [&](int blk) {
+    const uint32_t base = blk < b1 ? (uint32_t)blk * kAttnBlk : kOob / kAttnD;
+#pragma unroll
+    for (int kt = 0; kt < 2; ++kt) vsv[kt] = __builtin_amdgcn_raw_buffer_load_b128(vsr, (base + 16 * kt + 4 * o) * 4, 0, kNt);
+  };
+  // One round always, two from two query tiles up (8 tokens over 8192 rows, 257 blocks: 20.2 us against 20.9;
+  // 1 token 13.4 / 12.7); at three rounds and more the barriers cost what the merge does (16-node tree over 8k
+  // 25.3 / 25.2) and at eight more (8 tokens over 32k 35.0 / 30.5). The same for every split.
+  const bool shared = range.per <= (T > 1 ? 2 : 1) * kAttnWaves;
   fetch_k(b0 + wave);
-  fetch_v(b0 + wave);
+  if (shared) {
+    fetch_vs(b0 + wave);
+    fetch_vq(b0);
+  } else {
+    fetch_v(b0 + wave);
+  }
 
   // Q^T operand of MFMA (c, h): lane (i, o) holds row i of the tile, dims 64 c + 16 o + 8 h .. + 7. They sit
   // in LDS in lane order: in registers they and O^T did not fit beside the block in flight.
@@ -345,48 +394,52 @@ __global__ __launch_bounds__(64 * kAttnWaves, 1) void attn_split_kernel(AttnSpli
   }
   lds_barrier();
 
-  f32x4 acc[T][16];  // O^T tile e: dims 16 i' + e; lane (i, o), register r: row i, dim 64 o + 16 r + e
-  float m_i[T], l_i[T];
-#pragma unroll
-  for (int t = 0; t < T; ++t) {
-#pragma unroll
-    for (int e = 0; e < 16; ++e) acc[t][e] = f32x4{0.f, 0.f, 0.f, 0.f};
-    m_i[t] = -INFINITY;
-    l_i[t] = 0.f;
-  }
   const float sl2 = a.scale * kLog2e;
-  for (int blk = b0 + wave; blk < b1; blk += kAttnWaves) {
+  // Masked scores of block blk in log2 units, its V scales, and the K prefetch of the wave's next block
+  auto scores = [&](int blk, float (&sc)[T][8], float (&vf)[8], bool more) {
     // S^T = K8 Q^T for the block's two 16-key tiles (fp8 is exact in bf16): lane (i, o) gets keys
     // 16 kt + 4 o + r of row i; the key's scale multiplies the fp32 score
     f32x4 st[T][2];
 #pragma unroll
     for (int t = 0; t < T; ++t) st[t][0] = st[t][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    bf16x8 qc[T][2];
+#pragma unroll
+    for (int t = 0; t < T; ++t)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) qc[t][h] = *(const bf16x8*)(qs + (t * 8 + h) * 1024);
 #pragma unroll
     for (int c = 0; c < 4; ++c) {
+      bf16x8 qn[T][2];  // the next c's Q, read ahead of this one's MFMAs
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) qn[t][h] = *(const bf16x8*)(qs + ((t * 4 + (c < 3 ? c + 1 : c)) * 2 + h) * 1024);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const bf16x8 k0 = fp8x8_to_bf16(kraw[0][c][2 * h], kraw[0][c][2 * h + 1]);
         const bf16x8 k1 = fp8x8_to_bf16(kraw[1][c][2 * h], kraw[1][c][2 * h + 1]);
 #pragma unroll
         for (int t = 0; t < T; ++t) {
-          const bf16x8 q = *(const bf16x8*)(qs + ((t * 4 + c) * 2 + h) * 1024);
-          st[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, q, st[t][0], 0, 0, 0);
-          st[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, q, st[t][1], 0, 0, 0);
+          st[t][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k0, qc[t][h], st[t][0], 0, 0, 0);
+          st[t][1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k1, qc[t][h], st[t][1], 0, 0, 0);
         }
       }
+#pragma unroll
+      for (int t = 0; t < T; ++t)
+#pragma unroll
+        for (int h = 0; h < 2; ++h) qc[t][h] = qn[t][h];
       __builtin_amdgcn_sched_barrier(0);  // bounds the operands made ahead
     }
-    float kf[8], vf[8];
+    float kf[8];
 #pragma unroll
     for (int n = 0; n < 8; ++n) {
       kf[n] = __uint_as_float(ksv[n / 4][n % 4]) * sl2;
       vf[n] = __uint_as_float(vsv[n / 4][n % 4]);
     }
-    fetch_k(blk + kAttnWaves);
+    if (more) fetch_k(blk + kAttnWaves);
     const int64_t key0 = (int64_t)blk * kAttnBlk;
     const bool committed = key0 + kAttnBlk <= pos;  // uniform: no new key in the block, nothing to mask
-    // online softmax in log2 units: p = 2^(s - m) by v_exp_f32
-    float sc[T][8];
 #pragma unroll
     for (int t = 0; t < T; ++t)
 #pragma unroll
@@ -403,11 +456,124 @@ __global__ __launch_bounds__(64 * kAttnWaves, 1) void attn_split_kernel(AttnSpli
         for (int n = 0; n < 8; ++n) sc[t][n] = (seen >> (16 * (n / 4) + n % 4)) & 1u ? sc[t][n] : -INFINITY;
       }
     }
+  };
+  constexpr float kLazyMax = 48.f;
+
+  if (shared) {
+    // Rounds of four blocks, scores of one block to each wave; P^T meets in LDS at the row's common maximum and
+    // each wave makes its quarter of O^T over all four blocks, so nothing is left to merge.
+    char* const ps = (char*)lds + T * 8192;
+    float* const mw = (float*)(ps + kAttnWaves * T * 1024);
+    f32x4 oq[T][4];  // tile e: dims 64 wave + 4 i' + e; lane (i, o): row i, dims 64 wave + 16 o + 4 r + e
+    float m_r[T], l_r[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) oq[t][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+      m_r[t] = -INFINITY;
+      l_r[t] = 0.f;
+    }
+    // `more` is a constant at both uses: the last round issues no loads for a next one (one load instruction of a
+    // wave holds the CU's address unit for 16 cycles whether its lanes fetch or not)
+    auto round = [&](int blk0, bool more) {
+      float sc[T][8], vf[8];
+      scores(blk0 + wave, sc, vf, more);
+      if (more) fetch_vs(blk0 + kAttnWaves + wave);
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        const float mx = fmaxf(fmaxf(fmaxf(sc[t][0], sc[t][1]), fmaxf(sc[t][2], sc[t][3])),
+                               fmaxf(fmaxf(sc[t][4], sc[t][5]), fmaxf(sc[t][6], sc[t][7])));
+        const float mr = max_x32(max_x16(mx));
+        if (o == 0) mw[(t * 16 + i) * kAttnWaves + wave] = mr;
+      }
+      lds_barrier();
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        const float4 mv = *(const float4*)(mw + (t * 16 + i) * kAttnWaves);
+        const float mx = fmaxf(fmaxf(mv.x, mv.y), fmaxf(mv.z, mv.w));
+        if (mx > m_r[t] + kLazyMax) {  // the reference maximum and its restart: see below
+          m_r[t] = mx;
+          l_r[t] = 0.f;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) oq[t][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        const float m_safe = m_r[t] == -INFINITY ? 0.f : m_r[t];
+        uint32_t w[4];
+#pragma unroll
+        for (int n = 0; n < 8; n += 2) {
+          const float p0 = __builtin_amdgcn_exp2f(sc[t][n] - m_safe), p1 = __builtin_amdgcn_exp2f(sc[t][n + 1] - m_safe);
+          l_r[t] += p0 + p1;
+          w[n / 2] = pk_bf16(p0 * vf[n], p1 * vf[n + 1]);
+        }
+        *(uint4*)(ps + (wave * T + t) * 1024 + lane * 16) = make_uint4(w[0], w[1], w[2], w[3]);
+      }
+      lds_barrier();
+#pragma unroll
+      for (int b = 0; b < kAttnWaves; ++b) {
+        bf16x8 pb[T];
+#pragma unroll
+        for (int t = 0; t < T; ++t) pb[t] = *(const bf16x8*)(ps + (b * T + t) * 1024 + lane * 16);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const uint32_t sel = 0x0C0C0000u | ((4u + e) << 8) | (uint32_t)e;
+          uint32_t w[4];
+#pragma unroll
+          for (int n = 0; n < 4; ++n)
+            w[n] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(
+                                                    __builtin_amdgcn_perm(vq[b][2 * n + 1], vq[b][2 * n], sel), 1.f, false));
+          const bf16x8 va = __builtin_bit_cast(bf16x8, make_uint4(w[0], w[1], w[2], w[3]));
+#pragma unroll
+          for (int t = 0; t < T; ++t) oq[t][e] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(va, pb[t], oq[t][e], 0, 0, 0);
+        }
+      }
+      if (more) fetch_vq(blk0 + kAttnWaves);
+    };
+    int blk0 = b0;
+    for (; blk0 + kAttnWaves < b1; blk0 += kAttnWaves) round(blk0, true);
+    if (blk0 < b1) round(blk0, false);
+    // row sums over the octets, then over the waves (mw's reads are behind the last barrier)
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const float l = sum_x32(sum_x16(l_r[t]));
+      if (o == 0) mw[(t * 16 + i) * kAttnWaves + wave] = l;
+      // registers r <-> octets o transposed, so that a row's four lanes store 64 contiguous bytes
+      f32x4 v[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) v[e] = transpose_octets(oq[t][e]);
+      if (rvalid[t]) {
+        float* const part = a.acc_part + (head[t] * a.nsplit + s) * kAttnD + 64 * wave + 4 * o;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) *(float4*)(part + 16 * k) = make_float4(v[0][k], v[1][k], v[2][k], v[3][k]);
+      }
+    }
+    lds_barrier();
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      if (wave != 0 || o != 0 || !rvalid[t]) continue;
+      const float4 lv = *(const float4*)(mw + (t * 16 + i) * kAttnWaves);
+      a.m_part[head[t] * a.nsplit + s] = m_r[t];
+      a.l_part[head[t] * a.nsplit + s] = ((lv.x + lv.y) + lv.z) + lv.w;
+    }
+    return;
+  }
+
+  f32x4 acc[T][16];  // O^T tile e: dims 16 i' + e; lane (i, o), register r: row i, dim 64 o + 16 r + e
+  float m_i[T], l_i[T];
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[t][e] = f32x4{0.f, 0.f, 0.f, 0.f};
+    m_i[t] = -INFINITY;
+    l_i[t] = 0.f;
+  }
+  for (int blk = b0 + wave; blk < b1; blk += kAttnWaves) {
+    float sc[T][8], vf[8];
+    scores(blk, sc, vf, true);
+    // online softmax in log2 units: p = 2^(s - m) by v_exp_f32
     // Rows keep the maximum of their first block as the reference m (p, l and O^T are floats: any common scale
     // will do) until a key passes it by more than 2^kLazyMax. That key outweighs everything before it: 2^20
     // keys at the old maximum are 2^-28 of it, below fp32's last bit, so the row's sums restart from zero.
     // (Rescaling instead put O^T, which lives in AGPRs, through VGPRs and spilled.)
-    constexpr float kLazyMax = 48.f;
 #pragma unroll
     for (int t = 0; t < T; ++t) {
       float mx = fmaxf(fmaxf(fmaxf(sc[t][0], sc[t][1]), fmaxf(sc[t][2], sc[t][3])),
