@@ -1,4 +1,5 @@
-"""The verify GEMM at 1 to 16 rows: x staged in passes of eight rows, one strip in flight."""
+"""The verify GEMM at 1 to 16 rows: x staged through LDS beside the reduction ring and inside it, or read directly,
+with one strip and two in flight."""
 import pytest
 import torch
 
@@ -7,8 +8,10 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("sdt", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("N,K,slots", [
-    (16, 128, None),      # one strip, one wave, three padding groups
-    (48, 640, None),      # two waves, the second with one group
+    (16, 128, None),      # one strip, one wave, three padding groups; at 9 to 16 rows x read directly
+    (48, 640, None),      # two waves, the second with one group; likewise
+    (8208, 640, None),    # 513 strips: staged again
+    (12304, 3456, None),  # seven waves, four strips per workgroup: two in flight up to 8 rows
     (4112, 2048, None),   # 257 strips: one workgroup has two, three workgroups to a CU
     (528, 6144, 1),       # twelve waves
     (272, 17408, 3),      # 34 blocks over three slots: waves without a block

@@ -203,7 +203,7 @@ struct GemmArgs {
   int* am_cnt;            // arrival counter, zero between calls
   const int64_t* spec;    // [M] committed token + drafts, or null (argmax only)
   AcceptOut o;            // o.pred [M] always; the rest when spec != null
-  int xstage_off;         // byte offset of the activation staging area in dynamic LDS
+  int stage_off, shared;  // the activation staging area in dynamic LDS: its byte offset, or inside the ring
 };
 
 // q / d for q < 2^16 and 1 <= d < 2^15, magic = ceil(2^32 / d) (d == 1 has no 32-bit magic).
@@ -218,10 +218,9 @@ __device__ __forceinline__ int udiv_small(uint32_t q, int d, uint32_t magic) {
 namespace tr {
 
 // One accumulator tile element: (mt, lane, r) -> output row m = 16 mt + 4 (lane / 16) + r,
-// column n = 16 strip + lane % 16. XR = 8, 16 or 32: the most rows of x, staged in one pass of 8,
-// two of 8, or two of 16.
+// column n = 16 strip + lane % 16. XR = 8, 16 or 32: the most rows of x.
 //
-// Strips in flight. At one row tile a wave holds one strip, and each group's codes are reloaded for
+// Strips in flight (kInFlight). At one row tile a wave holds one strip (launch() has the exception), and each group's codes are reloaded for
 // the next strip as soon as the group is dequantized, so a group waits for its own load only and
 // the loads spread over the strip's MACs. Two strips in flight, each refilled after its last MAC,
 // sent the refill out in one burst with nothing to cover it but the other strip. Bound as before by
@@ -233,9 +232,9 @@ namespace tr {
 //   M = 8: 7.0 -> 6.3, 7.5 -> 6.5, 10.8 -> 10.0, 11.7 -> 10.6, 20.2 -> 18.7, 6.2 -> 6.0, 5.0 -> 4.7.
 // At two row tiles two strips stay: a group's MACs are twice as long and there are two groups to
 // a wave (M = 32 partials of 5120 x 6144 9.1 with two, 10.0 with one; 5120 x 17408 17.5 / 18.5).
-template <int XR, bool F16S>
+template <int XR, int kInFlight, bool F16S, bool kDirect>
 __global__ __launch_bounds__(768) void int4_gemm_kernel(GemmArgs a) {
-  constexpr int MT = XR > 16 ? 2 : 1, GW = MT == 1 ? 4 : 2, kInFlight = MT;
+  constexpr int MT = XR > 16 ? 2 : 1, GW = MT == 1 ? 4 : 2;
   // 16-byte aligned: the dynamic area follows the kernel's 776 bytes of static LDS, and the
   // ring's and staging area's 16-byte accesses stall when misaligned (SQ_LDS_UNALIGNED_STALL)
   extern __shared__ __attribute__((aligned(16))) float red[];  // [2][RB][W][MT][64][4]
@@ -284,21 +283,28 @@ __global__ __launch_bounds__(768) void int4_gemm_kernel(GemmArgs a) {
   uint4 xa[GW][MT][4];
   constexpr int kXL = XR == 8 ? 8 : 16;  // staging loads per wave: one per row (GW = 4), or per row pair (GW = 2)
   uint4 xv[kXL];                         // staged rows, held in VGPRs until they are written to LDS
-  {
+  if constexpr (kDirect) {
+#pragma unroll
+    for (int gw = 0; gw < GW; ++gw) {
+      const uint4* p = (const uint4*)(a.x + (size_t)min(lane & 15, a.M - 1) * a.K + min(gbase + gw, G - 1) * kGroup + 8 * (lane >> 4));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) xa[gw][0][j] = p[4 * j];
+    }
+  } else {
     // M <= 16: load the rows coalesced into VGPRs, write them to this wave's LDS staging area,
     // then read them back in the operand layout. In the operand layout itself consecutive lanes
     // would read different rows, each lane a separate cache access, which took 3-6 us for these
     // 8 KB per wave. Loading straight into LDS (buffer_load ... lds) lands no earlier and made the
-    // M = 8 layer set 0.8 us slower than this register round trip. Load t brings row t of the wave's four
-    // groups (lane l: group l / 16, 16-byte chunk (l % 16) ^ (t % 8)), so a call issues M loads, one per
-    // real row: every load instruction costs the CU's address unit the same 16 cycles whether
-    // its lanes fetch or not. The staging area holds row r of group gw at (r % 8 GW + gw) 256 bytes,
-    // chunk k of the row in 16-byte slot k ^ r % 8, so the rows read by one operand load fall in
-    // different LDS banks. Rows 8 to 15 follow rows 0 to 7 through the same 8 KB per wave. Lanes
-    // past row M - 1 take that row; their outputs are never stored. M = 9..16 loaded the operand
-    // layout directly before: M = 16 us, before -> now with one strip in flight, 5120 x 5120
-    // 9.4 -> 7.6, 7168 x 5120 9.8 -> 7.8, 16384 x 5120 14.2 -> 12.1, gate/up 22.4 -> 20.5,
-    // 5120 x 6144 partials 8.4 -> 7.3, 5120 x 17408 15.0 -> 12.5, 8192 x 2048 7.2 -> 5.7.
+    // M = 8 layer set 0.8 us slower than this register round trip. Up to 8 rows, load t brings row t of the
+    // wave's four groups (lane l: group l / 16, 16-byte chunk (l % 16) ^ row), so a call issues M loads, one per
+    // real row: every load instruction costs the CU's address unit the same 16 cycles whether its lanes fetch or
+    // not. The staging area holds the groups of a row side by side, chunk k in 16-byte slot k ^ row, so the 16 rows
+    // read by one operand load fall in different LDS banks. 9 to 16 rows: load t brings rows 2 (t % 8) and + 1 of
+    // two groups, and the two pairs of groups follow each other through the same 8 KB per wave (eight rows after
+    // eight instead read half the lanes' operands twice). Lanes past row M - 1 take that row; their outputs are
+    // never stored. 9 to 16 rows loaded the operand layout directly before: M = 16 us, before -> now with one strip
+    // in flight, 5120 x 5120 9.4 -> 7.4, gate/up 34816 x 5120 22.4 -> 20.7, 8192 x 5120 9.8 -> 8.2, partials of
+    // 5120 x 6144 8.2 -> 7.1 and of 5120 x 17408 13.6 -> 12.4.
     //
     // M = 17..32 (two row tiles, two groups per wave): load u brings rows 2u and 2u + 1 (lanes
     // 0-31 and 32-63; lane l: group (l / 16) % 2, chunk (l % 16) ^ (row % 16)), all 16 loads
@@ -308,11 +314,13 @@ __global__ __launch_bounds__(768) void int4_gemm_kernel(GemmArgs a) {
     const auto xrs = __builtin_amdgcn_make_buffer_rsrc((void*)a.x, (short)0, a.M * a.K * 2, 0x00020000);
     const int lk = lane & 15;
     if constexpr (MT == 1) {
-      const int g = min(gbase + (lane >> 4), G - 1);
+      // xv[t]: XR == 8: row t of the four groups; XR == 16: rows 2 (t % 8) and + 1 of group pair t / 8
 #pragma unroll
       for (int t = 0; t < XR; ++t) {
-        if (t >= a.M) continue;
-        const int off = (t * a.K + g * kGroup) * 2 + (lk ^ (t & 7)) * 16;
+        if ((XR == 8 ? t : 2 * (t & 7)) >= a.M) continue;
+        const int row = XR == 8 ? t : min(2 * (t & 7) + (lane >> 5), a.M - 1);
+        const int g = min(gbase + (XR == 8 ? lane >> 4 : 2 * (t >> 3) + ((lane >> 4) & 1)), G - 1);
+        const int off = (row * a.K + g * kGroup) * 2 + ((lk ^ row) & 15) * 16;
         const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(xrs, off, 0, 0);
         xv[t] = make_uint4(v.x, v.y, v.z, v.w);
       }
@@ -339,27 +347,26 @@ __global__ __launch_bounds__(768) void int4_gemm_kernel(GemmArgs a) {
 #pragma unroll
   for (int h = 0; h < kInFlight; ++h) load_strip<GW>(buf[h], rsrc, active ? strip_off(r0 + h) : oob, lane_off, sm_voff);
   TLM(3);
-  {
+  if constexpr (!kDirect) {
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"(kInFlight * (GW + 1)) : "memory");  // the staging loads have landed
     TLM(2);
-    char* stage = (char*)red + a.xstage_off + wave * 8192;
+    char* stage = (char*)red + a.stage_off + wave * 8192;
     const int i = lane & 15;
     if constexpr (MT == 1) {
+      constexpr int P = XR / 8, PG = GW / P;  // passes, groups of each
+      const int rs = min(i, a.M - 1);
 #pragma unroll
-      for (int p = 0; p < XR / 8; ++p) {
+      for (int p = 0; p < P; ++p) {
 #pragma unroll
         for (int t = 0; t < 8; ++t) {
-          if (8 * p + t >= a.M) continue;
-          *(uint4*)(stage + t * 1024 + lane * 16) = xv[8 * p + t];  // lane l: chunk l % 16 of group l / 16
+          if (P * t >= a.M) continue;
+          *(uint4*)(stage + t * 1024 + lane * 16) = xv[8 * p + t];
         }
-        const int rs = p ? min(i, a.M - 1) - 8 : min(min(i, 7), a.M - 1);  // staged row
-        if (p == 0 || i >= 8) {
 #pragma unroll
-          for (int gw = 0; gw < GW; ++gw)
+        for (int h = 0; h < PG; ++h)
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-              xa[gw][0][j] = *(const uint4*)(stage + (rs * GW + gw) * 256 + ((4 * j + (lane >> 4)) ^ rs) * 16);
-        }
+          for (int j = 0; j < 4; ++j)
+            xa[PG * p + h][0][j] = *(const uint4*)(stage + (rs * PG + h) * 256 + (((4 * j + (lane >> 4)) ^ rs) & 15) * 16);
       }
     } else {
 #pragma unroll
@@ -376,8 +383,8 @@ __global__ __launch_bounds__(768) void int4_gemm_kernel(GemmArgs a) {
           }
         }
       }
-      lds_barrier();  // every wave's staging reads before any ring write
     }
+    if (MT == 2 || a.shared) lds_barrier();  // every wave's staging reads before any ring write
   }
 
   // Xa[mt] = sum of x over group gbase + lane / 16 for row 16 mt + lane % 16 (the A operand of
@@ -652,7 +659,7 @@ namespace {
 constexpr int kCUs = 256;          // MI355X compute units
 
 constexpr int kWavesPerCU = 12;    // occupancy of the GEMM kernel (about 150 VGPRs per lane)
-constexpr size_t kLdsBudget = 64 * 1024;  // LDS of the reduction ring
+constexpr size_t kLdsBudget = 64 * 1024;  // LDS of the reduction ring where the staging area lies beside it
 constexpr size_t kLdsMax = 152 * 1024;    // dynamic LDS of one workgroup: gfx950's 160 KB less the kernel's static LDS
 
 struct Plan {
@@ -725,35 +732,36 @@ bool make_plan(int N, int K, int M, int S_req, int R_req, Plan* p) {
   return true;
 }
 
-template <int XR, bool F16S>
+template <int XR, int kInFlight, bool F16S, bool kDirect = false>
 hipError_t launch_t(GemmArgs a, const Plan& p, hipStream_t stream) {
   constexpr int MT = XR > 16 ? 2 : 1;
   const dim3 grid(p.grid_n * p.S), block(64 * p.W);
   const size_t per_strip = (size_t)p.W * MT * 256 * sizeof(float);
-  // Ring budget: at one row tile 64 KB (the staging area takes the rest). The two-tile staging
-  // area shares the ring (it is dead before the first partial is written), which shares the CU's
-  // LDS among the workgroups the plan puts on one CU, so larger batches never cost occupancy.
-  constexpr bool kShared = MT == 2;
+  // Several workgroups on a CU share its LDS, and there the ring takes the staging area's place (staging is over
+  // before the first partial is written), so that neither costs occupancy: side by side they took 64 KB at W = 4,
+  // two workgroups on a CU instead of three (M = 8: gate/up 24576 x 1024 9.7 us -> 6.7, 8192 x 3072 8.5 -> 7.3,
+  // 34816 x 2048 11.2 -> 10.2). One workgroup to a CU keeps them apart, without the barrier between them (M = 8:
+  // gate/up 34816 x 5120 18.4 us against 19.8, 5120 x 17408 11.4 against 12.2). At two row tiles they always share.
   const int wg_per_cu = p.W >= kWavesPerCU ? 1 : kWavesPerCU / p.W;
-  int rb = (int)((!kShared ? kLdsBudget : kLdsMax / wg_per_cu) / (2 * per_strip));
+  a.shared = MT == 2 || wg_per_cu > 1;
+  const int rb = (int)((a.shared ? kLdsMax / wg_per_cu : kLdsBudget) / (2 * per_strip));
   a.RB = rb < 1 ? 1 : (rb > 4 ? 4 : rb);
-  const size_t ring = 2 * a.RB * per_strip;
-  const size_t stage = (size_t)p.W * 8192;
-  a.xstage_off = kShared ? 0 : (int)ring;
-  const size_t lds = kShared ? (ring > stage ? ring : stage) : ring + stage;
+  const size_t ring = 2 * a.RB * per_strip, stage = (size_t)p.W * 8192;
+  a.stage_off = a.shared ? 0 : (int)ring;
+  const size_t lds = !a.shared ? ring + stage : ring > stage ? ring : stage;
   {
-    // staging + ring, or a ring over 64 KB, exceed the default 64 KB of dynamic LDS: raise this
+    // staging or a ring over 64 KB exceeds the default dynamic LDS: raise this
     // kernel's limit once
     static bool raised = false;
     if (!raised) {
-      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&int4_gemm_kernel<XR, F16S>),
+      const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&int4_gemm_kernel<XR, kInFlight, F16S, kDirect>),
                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsMax);
       if (e != hipSuccess) return e;
       raised = true;
     }
     if (lds > kLdsMax) return hipErrorInvalidValue;
   }
-  hipLaunchKernelGGL((int4_gemm_kernel<XR, F16S>), grid, block, lds, stream, a);
+  hipLaunchKernelGGL((int4_gemm_kernel<XR, kInFlight, F16S, kDirect>), grid, block, lds, stream, a);
   return hipGetLastError();
 }
 
@@ -790,9 +798,20 @@ hipError_t launch_wide_gw(const GemmArgs& a, int R_req, int scale_dtype, hipStre
 
 hipError_t launch(const GemmArgs& a, const Plan& p, int scale_dtype, hipStream_t stream) {  // NOLINT
   const bool f16 = scale_dtype == 1;
-  if (a.M > 16) return f16 ? launch_t<32, true>(a, p, stream) : launch_t<32, false>(a, p, stream);
-  if (a.M <= 8) return f16 ? launch_t<8, true>(a, p, stream) : launch_t<8, false>(a, p, stream);
-  return f16 ? launch_t<16, true>(a, p, stream) : launch_t<16, false>(a, p, stream);
+  if (a.M > 16) return f16 ? launch_t<32, 2, true>(a, p, stream) : launch_t<32, 2, false>(a, p, stream);
+  // 9 to 16 rows over one or two waves: where at most two workgroups meet on a CU, the few loads of x in operand
+  // layout cost less than the trip through LDS (M = 16, us: 1600 x 512 4.0 against 4.7, 512 x 1024 3.8 / 4.2,
+  // 8192 x 1024 5.4 / 5.5); more share its address unit, and the staged kernel leads (15360 x 1024 7.4 / 6.2,
+  // 24576 x 1024 9.9 / 7.8, 34816 x 1024 10.8 / 9.5).
+  if (a.M > 8 && p.W <= 2 && p.grid_n * p.S <= 2 * kCUs)
+    return f16 ? launch_t<16, 1, true, true>(a, p, stream) : launch_t<16, 1, false, true>(a, p, stream);
+  if (a.M > 8) return f16 ? launch_t<16, 1, true>(a, p, stream) : launch_t<16, 1, false>(a, p, stream);
+  // Seven or eight waves are all of a CU's (two workgroups don't fit), too few for one strip each to cover the
+  // memory latency of a long run of strips: two in flight (M = 1 / 8, us, one -> two: gate/up 15360 x 3456
+  // 8.1 / 8.5 -> 7.9 / 8.2, 34816 x 3456 14.5 / 15.2 -> 14.1 / 14.9; at two strips per workgroup one stays better,
+  // 8192 x 3456 5.5 / 6.0 against 6.0 / 6.4).
+  if (p.W >= 7 && p.W <= 8 && p.R >= 4) return f16 ? launch_t<8, 2, true>(a, p, stream) : launch_t<8, 2, false>(a, p, stream);
+  return f16 ? launch_t<8, 1, true>(a, p, stream) : launch_t<8, 1, false>(a, p, stream);
 }
 
 }  // namespace
