@@ -337,14 +337,14 @@ def config4_tree_step(torch, dev, model, reps=10, M=32):
     t = sum(times) / len(times)
     return {"ms_per_step": round(t * 1e3, 3), "M": M, "replays": reps,
             "accepted_depth": sorted(set(accepted)), "planted_depth": len(path) - 1,
-            "note": "one hipGraph: 257 int4 GEMMs at M=32 (the 64 gate/up GEMMs then slot_sum_kernel for their two K slots and silu), tree GDN steps (per-node state, 32 snapshot slots), "
+            "note": "one hipGraph: 257 int4 GEMMs at M=32 (the 64 gate/up with silu_mul in the epilogue), tree GDN steps (per-node state, 32 snapshot slots), "
                     "ancestor-masked FP8 attention over 8192 live tokens, lm_head 248320x5120 writing logits, tree "
                     "accept, commit of KV rows/scales (4 launches) and conv rings (1 launch); node tokens planted "
                     "along the deepest root path, each replay from the same restored state"}
 
 
 TL_MARKS = {0: "entry", 1: "launch constants", 21: "activation loads issued", 22: "past the ordering barrier",
-            3: "first two strips issued", 2: "activations staged",
+            3: "first strips issued", 2: "activations staged",
             4: "prologue end", 5: "strip 0 MACs", 6: "strip 1 MACs", 7: "strip 2 MACs", 8: "strip 3 MACs",
             9: "strip 4 MACs", 10: "strip 5 MACs", 16: "batch reduced (last)", 20: "strip loop exit",
             19: "slot-sum arrival (K slots > 1)", 23: "slot sum done (last arriver)"}

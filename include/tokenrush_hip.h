@@ -71,13 +71,14 @@ int tr_int4_gemm_noalloc(const void* x, const void* packed, void* out, int M, in
  * tr_pack_int4_pairs; out bf16 [M, N/2] = silu(bf16(x . gate^T)) * bf16(x . up^T), bit for bit what
  * tr_int4_gemm followed by tr_silu_mul produce. N % 32 == 0; workspace as for tr_int4_gemm.
  * Replaces: silu_mul(gate_up(n)) (tokenrush/model.py:156-160, tokenrush/fused.py:67-87) in one launch, or
- * two when the plan takes more than one K slot (M > 16 at K = 5120): the K slots' partials into the
+ * two when K takes more than one slot (K > 6144, at M > 16 K > 5120): the K slots' partials into the
  * workspace, then their in-order sum and the activation. */
 int tr_int4_gemm_silu(const void* x, const void* packed, void* out, void* workspace, size_t workspace_bytes, int M,
                       int N, int K, int group, int scale_dtype, void* stream);
 
 /* The default tiling of an N x K weight for M rows: S K-slots, W waves and R strips per
- * workgroup. Depends on M only through M > 16. Host only, no GPU call. */
+ * workgroup. Depends on M only through M > 16. At M > 16 and 24 < K / 128 <= 40 it is what explicit slots and
+ * workspace sizes go by; out mode with default slots runs there in one slot. Host only, no GPU call. */
 int tr_gemm_plan(int N, int K, int M, int* S, int* W, int* R);
 
 /* fp32 slots a partial-mode call writes for an N x K weight at M rows (-1: unsupported shape).

@@ -38,7 +38,7 @@
 // Before, four waves converted each block into LDS together (two barriers and a transposed write per block)
 // and then held 16 query rows each: 2.4 us per 32 keys of a CU, whatever the rows. Split + combine, us
 // (24 / 4 heads): 1 token over 100k rows 87 -> 42, 4 tokens 90 -> 46 (208 MB, 4.9 TB/s in the split kernel),
-// 8 tokens 93 -> 54; over 8k rows 15.7 -> 12.6, 19.0 -> 16.4, 22.6 -> 21.0; a 32-node tree over 8k 37 -> 29.
+// 8 tokens 93 -> 54; over 8k rows 15.7 -> 12.6, 19.0 -> 16.2, 22.6 -> 20.2; a 32-node tree over 8k 37 -> 29.
 // Measured and not kept: a second block of K and V in flight in registers (M = 8 over 8k 22.3 us, 100k 61.6;
 // the copies cost more than the wait); key splits not rounded to four blocks (22.9 us at 8k); partial rows
 // stored whole through a transposing LDS read (22.6 us; the merge of a 16-row tile costs 2.3 us either way).

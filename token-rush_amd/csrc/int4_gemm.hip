@@ -13,8 +13,8 @@
 //   * An MFMA chain against a ones operand gives X = sum(x) per row and group, and the group
 //     result is  s * E + (mn - 128 s) * X  in fp32, applied once per group.
 //
-// Rows of x beyond M are padding lanes (they load row M-1 and are never stored), so every
-// output row is computed by the same instructions for every M of one row-tile count: row i
+// Rows of x beyond M are padding lanes (never stored), so every
+// output row is computed by the same arithmetic for every M of one row-tile count: row i
 // of an M = 1 call is bit-identical to row i of an M = 16 call (the property the reference's
 // tests/test_marlin.py:42-52 checks for Marlin), and likewise within M = 17..32.
 //

@@ -10,11 +10,11 @@ design, not Marlin:
   codes in the order one wave's 16-byte loads consume them, then the 16 rows' (scale, min)
   pairs for the four groups (16 bytes per row). A strip is one contiguous stream of whole
   128-byte lines;
-* every M in 1..16 runs the same instructions (rows beyond M are padding lanes), so each
+* every M in 1..16 runs the same arithmetic (rows beyond M are padding lanes), so each
   output row is bit-identical for every M, as Marlin's is (reference test_marlin.py:42-52);
   the same holds within M = 17..32;
 * no locks: split-K inside a workgroup is reduced through LDS in a fixed order; split-K
-  across workgroups (K = 17408, or M > 16) writes fp32 slots, which mul_partial returns as
+  across workgroups (K = 17408, or partials) writes fp32 slots, which mul_partial returns as
   [S, M, N] and mul reduces in the last-arriving workgroup through the workspace.
 
 API (same names and argument meaning as marlin.py): ext, available, pack, unpack,
