@@ -26,9 +26,9 @@
 //   Row maxima need two permlane swaps, row sums are made after the loop. After the last block the waves'
 //   (m, l, O^T) meet in LDS.
 // A split of one or two rounds of four blocks does not merge O^T: the waves' P^T meet in LDS instead, and each
-// wave makes a quarter of the dims over all of a round's blocks (attn_split_kernel's `shared`). The merge of
-// three tiles was 3 of 9 us there; with the last round's empty prefetches gone and O^T transposed over the octets,
-// so that its stores are 64 contiguous bytes a row, split + combine over 1k rows went, us: 1 token 9.5 -> 8.5,
+// wave makes a quarter of the dims over all of a round's blocks (attn_split_kernel's `shared`). That alone
+// took 1.5 us off 8 tokens over 1k rows; with the last round's empty prefetches gone and O^T transposed over the
+// octets, so that its stores are 64 contiguous bytes a row, split + combine over 1k rows went, us: 1 token 9.5 -> 8.5,
 // 8 tokens 15.0 -> 12.9, a 32-node tree 20.5 -> 17.8. What is left of the split at 8 tokens over 8100 rows (9.1 us
 // from entry): 4.4 until K, V and Q are there (17 MB), 2.7 for scores, probabilities and O^T, 1.9 for 12.6 MB of
 // partials.
